@@ -573,6 +573,7 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
     constexpr int EPB = C::EPB, LC = C::LC, BLOCK = C::BLOCK, FXN = C::FXN, JF = C::JF;
     constexpr int NQ = RhsSmem<DIM, NP, BLEND, QNS3, FB, GEN, AXI>::NQ;
     static_assert(!AXI || (GEN && DIM == 2), "axisymmetric meshes are quadrilateral meshes");
+    constexpr bool DIVF = DIM == 3 && NP >= 6;   // the division form of the two-point flux (dg_physics.h)
     constexpr int MC = DIM * DIM;   // adjugate entries per node (general geometry)
     auto &sM = S.M;
     (void)sM;
@@ -928,7 +929,7 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
             }
             const NodeQ<DIM> q1 = node_quants<DIM>(g1, P);
             const NodeQ<DIM> q2 = node_quants<DIM>(g2, P);
-            two_point_flux_v<DIM, true>(nvec, norml2_v<DIM>(nvec), q1, q2, g1, g2, P, quirk3d, F);
+            ec_flux<DIM, true>(nvec, norml2_v<DIM>(nvec), q1, q2, P, quirk3d, F);
             if constexpr (AXI) {
                 // flux_num *= r (DGSEMIntegrator.cpp:190-205), the r of the
                 // first element's node on both sides
@@ -1013,8 +1014,16 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
         const NodeQ<DIM> q1 = node_quants<DIM>(s1, P);
         const NodeQ<DIM> q2 = node_quants<DIM>(s2, P);
         double F[NV];
-        if (A.ec) two_point_flux<DIM, false>(r, nr, nr, q1, q2, nullptr, nullptr, P, false, F);
-        else two_point_flux<DIM, true>(r, nr, nr, q1, q2, s1, s2, P, quirk3d, F);
+        if constexpr (DIVF) {
+            if (A.ec) two_point_flux<DIM, false>(r, nr, nr, q1, q2, nullptr, nullptr, P, false, F);
+            else two_point_flux<DIM, true>(r, nr, nr, q1, q2, s1, s2, P, quirk3d, F);
+        } else {
+            double nvec[DIM];
+#pragma unroll
+            for (int d = 0; d < DIM; d++) nvec[d] = (d == r) ? nr : 0.0;
+            if (A.ec) ec_flux<DIM, false>(nvec, nr, q1, q2, P, false, F);
+            else ec_flux<DIM, true>(nvec, nr, q1, q2, P, quirk3d, F);
+        }
 #pragma unroll
         for (int v = 0; v < NV; v++) {
             double d;
@@ -1053,6 +1062,9 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
 
     for (int r = 0; r < DIM; r++) {
         const double nr = A.geo.nrm[r];
+        double nvr[DIM];   // the box's metric vector of direction r
+#pragma unroll
+        for (int d = 0; d < DIM; d++) nvr[d] = (d == r) ? nr : 0.0;
         if (PREFETCH && r == DIM - 1 && act) {
             // inputs of the final assembly, in flight during the last direction
 #pragma unroll
@@ -1086,7 +1098,7 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
                         double mm[DIM];
 #pragma unroll
                         for (int d = 0; d < DIM; d++) mm[d] = (sM[ej][DIM * r + d][row_slot<DIM, NP>(na)] + sM[ej][DIM * r + d][row_slot<DIM, NP>(nb)]) * 0.5;
-                        two_point_flux_v<DIM, false>(mm, 0.0, qa, qb, nullptr, nullptr, P, false, F);
+                        ec_flux<DIM, false>(mm, 0.0, qa, qb, P, false, F);
                         if constexpr (AXI) {
                             // f *= r_hat, r at the pair's midpoint (DGSEMIntegrator.cpp:272-292)
                             const double rh = (sR[ej][na] + sR[ej][nb]) * 0.5;
@@ -1094,7 +1106,8 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
                             for (int v = 0; v < NV; v++) F[v] *= rh;
                         }
                     } else {
-                        two_point_flux<DIM, false>(r, nr, nr, qa, qb, nullptr, nullptr, P, false, F);
+                        if constexpr (DIVF) two_point_flux<DIM, false>(r, nr, nr, qa, qb, nullptr, nullptr, P, false, F);
+                        else ec_flux<DIM, false>(nvr, nr, qa, qb, P, false, F);
                     }
 #pragma unroll
                     for (int v = 0; v < NV; v++) sF[ej][v][lc * NPAIR + p] = F[v];
@@ -1116,11 +1129,8 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
                     }
                     const int na = line_node<DIM, NP>(r, l0 + lc, i);
                     const int nb = line_node<DIM, NP>(r, l0 + lc, i + 1);
-                    double s1[NV], s2[NV];
                     NodeQ<DIM> qa, qb;
-#pragma unroll
-                    for (int v = 0; v < NV; v++) { s1[v] = sU[ej][v][row_slot<DIM, NP>(na)]; s2[v] = sU[ej][v][row_slot<DIM, NP>(nb)]; }
-                    qa.rho = s1[0]; qb.rho = s2[0];
+                    qa.rho = sU[ej][0][row_slot<DIM, NP>(na)]; qb.rho = sU[ej][0][row_slot<DIM, NP>(nb)];
 #pragma unroll
                     for (int d = 0; d < DIM; d++) { qa.v[d] = sQ[ej][d][row_slot<DIM, NP>(na)]; qb.v[d] = sQ[ej][d][row_slot<DIM, NP>(nb)]; }
                     qa.beta = sQ[ej][DIM][row_slot<DIM, NP>(na)]; qb.beta = sQ[ej][DIM][row_slot<DIM, NP>(nb)];
@@ -1132,7 +1142,7 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
                         double nv2[DIM];
 #pragma unroll
                         for (int d = 0; d < DIM; d++) nv2[d] = sn[d];
-                        two_point_flux_v<DIM, true>(nv2, norml2_v<DIM>(nv2), qa, qb, s1, s2, P, quirk3d, F);
+                        ec_flux<DIM, true>(nv2, norml2_v<DIM>(nv2), qa, qb, P, quirk3d, F);
                         if constexpr (AXI) {
                             // flux_num *= mid_r (DGSEMIntegrator.cpp:1030-1032, 1110-1112)
                             const double rh = (sR[ej][na] + sR[ej][nb]) * 0.5;
@@ -1140,7 +1150,17 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
                             for (int v = 0; v < NV; v++) F[v] *= rh;
                         }
                     } else {
-                        two_point_flux<DIM, true>(r, sSub[r][i], sSub[r][i], qa, qb, s1, s2, P, quirk3d, F);
+                        if constexpr (DIVF) {
+                            double s1[NV], s2[NV];
+#pragma unroll
+                            for (int v = 0; v < NV; v++) { s1[v] = sU[ej][v][row_slot<DIM, NP>(na)]; s2[v] = sU[ej][v][row_slot<DIM, NP>(nb)]; }
+                            two_point_flux<DIM, true>(r, sSub[r][i], sSub[r][i], qa, qb, s1, s2, P, quirk3d, F);
+                        } else {
+                            double nv2[DIM];
+#pragma unroll
+                            for (int d = 0; d < DIM; d++) nv2[d] = (d == r) ? sSub[r][i] : 0.0;
+                            ec_flux<DIM, true>(nv2, sSub[r][i], qa, qb, P, quirk3d, F);
+                        }
                     }
 #pragma unroll
                     for (int v = 0; v < NV; v++) sF[ej][v][slot] = F[v];

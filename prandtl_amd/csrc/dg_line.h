@@ -23,100 +23,10 @@
 // value, as in k_rhs.  Summation order differs from k_rhs (per direction, then
 // over directions), so the two kernels agree to rounding, not bitwise; every
 // launch of this kernel rounds identically.
-//
-// The two-point flux here is ChandrashekarFlux::ComputeVolumeFlux /
-// ComputeFaceFlux (ChandrashekarFlux.cpp:11-161) rearranged to two
-// reciprocals per pair instead of four divisions:
-//   - the log mean is formed as num/den (series branch: 52.5 s t^3 over the
-//     series denominator; log branch: (y-x) over log(y/x)), so rho_ln needs
-//     one reciprocal of den;
-//   - 1/beta_ln = den_b/num_b and p_hat = (rho1+rho2)/(2(beta1+beta2)) share
-//     one reciprocal of num_b (beta1+beta2);
-//   - the energy flux rho_ln Vn (... + p_hat/rho_ln) is rho_ln Vn (...) +
-//     Vn p_hat (the distributive law), so 1/rho_ln is never formed.
-// Each reciprocal is v_rcp_f64 refined by two Newton-Raphson steps (the
-// textbook iteration r <- r + r(1 - x r)), within an ulp or two of the
-// correctly rounded value; the log branch keeps the IEEE quotient y/x inside
-// the logarithm.  The results differ from the reference's by rounding only.
 #pragma once
 #include "dg_device.h"
 
 namespace prandtl {
-
-// Log mean LM(x, y) = num / den, the branches of ComputeLogMean
-// (BasicOperations.cpp:6-12, eps 1e-4) as in logmean(): u = d^2/s^2.
-__device__ __forceinline__ void lm_parts(double x, double y, double &num, double &den)
-{
-    const double d = y - x, s = y + x;
-    const double q = d * d, t = s * s;
-    if (q < 1e-4 * t) {
-        num = 52.5 * s * (t * t * t);
-        den = lm_series_den(q, t);
-    } else {
-        num = d;
-        den = log(y / x);
-    }
-}
-
-// Chandrashekar two-point flux for the normal nr e_r (see the file header).
-// DISS = false: the volume flux; DISS = true: the face flux with the jumps of
-// s1, s2 and dissipation scaled by |nr|; quirk3d: the 3-D energy term of
-// ChandrashekarFlux.cpp:131 as written.
-template <int DIM, bool DISS>
-__device__ __forceinline__ void ec_flux(int r, double nr, const NodeQ<DIM> &a, const NodeQ<DIM> &b,
-                                        const double *s1, const double *s2, const Phys &P, bool quirk3d,
-                                        double *F)
-{
-    double nrh, drh, nbt, dbt;
-    lm_parts(a.rho, b.rho, nrh, drh);
-    lm_parts(a.beta, b.beta, nbt, dbt);
-    const double rho_ln = nrh * rcp_nr(drh);
-    const double bsum = a.beta + b.beta;
-    const double rb = rcp_nr(nbt * bsum);
-    const double ibeta_ln = dbt * bsum * rb;
-    const double rsum = a.rho + b.rho;
-    const double p_hat = 0.5 * rsum * nbt * rb;
-    double vm[DIM];
-    double h = 0.0, diss = 0.0;
-    const double drho = b.rho - a.rho;
-    const double rho_mean = 0.5 * rsum;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        vm[d] = 0.5 * (a.v[d] + b.v[d]);
-        const double hd = -0.25 * (a.v[d] * a.v[d] + b.v[d] * b.v[d]) + vm[d] * vm[d];
-        h = (d == 0) ? hd : h + hd;
-        if (DISS) {
-            const double dv = b.v[d] - a.v[d];
-            const double t0 = 0.5 * drho * a.v[d] * b.v[d];
-            const double dd = (DIM == 3 && d == 2 && quirk3d) ? t0 + rho_mean * dv + vm[d]
-                                                              : t0 + rho_mean * dv * vm[d];
-            diss = (d == 0) ? dd : diss + dd;
-        }
-    }
-    double vr = vm[0];
-#pragma unroll
-    for (int d = 1; d < DIM; d++)
-        if (d == r) vr = vm[d];
-    const double Vn = vr * nr;
-    h += 0.5 * ibeta_ln * P.gm1i;
-    const double rVn = rho_ln * Vn;
-    F[0] = rVn;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        const double mom = Vn * (rho_ln * vm[d]);
-        F[1 + d] = (d == r) ? mom + p_hat * nr : mom;
-    }
-    F[DIM + 1] = rVn * h + Vn * p_hat;
-    if (DISS) {
-        diss += 0.5 * drho * P.gm1i * ibeta_ln + 0.5 * rho_mean * P.gm1i * (b.ibeta - a.ibeta);
-        const double lam = (a.lam < b.lam) ? b.lam : a.lam;
-        const double hl = 0.5 * lam * fabs(nr);
-        F[0] = F[0] - hl * (s2[0] - s1[0]);
-#pragma unroll
-        for (int d = 0; d < DIM; d++) F[1 + d] = F[1 + d] - hl * (s2[1 + d] - s1[1 + d]);
-        F[DIM + 1] = F[DIM + 1] - hl * diss;
-    }
-}
 
 constexpr int line_epb(int TE)
 {
@@ -263,6 +173,7 @@ __attribute__((amdgpu_waves_per_eu((LCfg<DIM, NP>::WAVES)))) k_rhs_ln(const KArg
             return pb + m * ps;
     };
     const double nr = r == 0 ? A.geo.nrm[0] : (r == 1 ? A.geo.nrm[1] : A.geo.nrm[2]);
+    const double nvec[3] = {r == 0 ? nr : 0.0, r == 1 ? nr : 0.0, r == 2 ? nr : 0.0};
 
     // Every global load of the start is issued on every path, the workgroup's
     // nodes first.  Loads complete in issue order, so the node phase then
@@ -490,13 +401,13 @@ __attribute__((amdgpu_waves_per_eu((LCfg<DIM, NP>::WAVES)))) k_rhs_ln(const KArg
             const NodeQ<DIM> qn = node_quants<DIM>(pn, P);
             double F[NV];
             if (side) {
-                if (A.ec) ec_flux<DIM, false>(r, nr, qo, qn, nullptr, nullptr, P, false, F);
-                else ec_flux<DIM, true>(r, nr, qo, qn, s1, s2, P, quirk3d, F);
+                if (A.ec) ec_flux<DIM, false>(nvec, nr, qo, qn, P, false, F);
+                else ec_flux<DIM, true>(nvec, nr, qo, qn, P, quirk3d, F);
 #pragma unroll
                 for (int v = 0; v < NV; v++) acc[NP - 1][v] = aface * (A.parabolic ? (-F[v] + fvn[v]) : -F[v]);
             } else {
-                if (A.ec) ec_flux<DIM, false>(r, nr, qn, qo, nullptr, nullptr, P, false, F);
-                else ec_flux<DIM, true>(r, nr, qn, qo, s1, s2, P, quirk3d, F);
+                if (A.ec) ec_flux<DIM, false>(nvec, nr, qn, qo, P, false, F);
+                else ec_flux<DIM, true>(nvec, nr, qn, qo, P, quirk3d, F);
 #pragma unroll
                 for (int v = 0; v < NV; v++) acc[0][v] = aface * (A.parabolic ? (F[v] - fvn[v]) : F[v]);
             }
@@ -523,7 +434,7 @@ __attribute__((amdgpu_waves_per_eu((LCfg<DIM, NP>::WAVES)))) k_rhs_ln(const KArg
                 for (int d = 0; d < DIM; d++) qb.v[d] = sQ(el, d, nb);
                 qb.beta = sQ(el, DIM, nb);
                 double F[NV];
-                ec_flux<DIM, false>(r, nr, qa, qb, nullptr, nullptr, P, false, F);
+                ec_flux<DIM, false>(nvec, nr, qa, qb, P, false, F);
                 const double dab = cv * A.tab.Dh2[a * MAXNP + b], dba = cv * A.tab.Dh2[b * MAXNP + a];
 #pragma unroll
                 for (int v = 0; v < NV; v++) {
@@ -543,7 +454,8 @@ __attribute__((amdgpu_waves_per_eu((LCfg<DIM, NP>::WAVES)))) k_rhs_ln(const KArg
                     for (int d = 0; d < DIM; d++) qe.v[d] = sQ(el, d, ne);
                     qe.beta = sQ(el, DIM, ne);
                     double g[NV];
-                    ec_flux<DIM, false>(1, A.geo.nrm[1], qa, qe, nullptr, nullptr, P, false, g);
+                    const double n1[3] = {0.0, A.geo.nrm[1], 0.0};
+                    ec_flux<DIM, false>(n1, A.geo.nrm[1], qa, qe, P, false, g);
 #pragma unroll
                     for (int b = a + 1; b < NP; b++) {
                         const double dba = cv * A.tab.Dh2[b * MAXNP + a];
@@ -564,11 +476,8 @@ __attribute__((amdgpu_waves_per_eu((LCfg<DIM, NP>::WAVES)))) k_rhs_ln(const KArg
 #pragma unroll
                 for (int i = 0; i < NP - 1; i++) {
                     const int na = lnode(i), nb = lnode(i + 1);
-                    double s1[NV], s2[NV];
-#pragma unroll
-                    for (int v = 0; v < NV; v++) { s1[v] = sU(el, v, na); s2[v] = sU(el, v, nb); }
                     NodeQ<DIM> qa, qb;
-                    qa.rho = s1[0]; qb.rho = s2[0];
+                    qa.rho = sU(el, 0, na); qb.rho = sU(el, 0, nb);
 #pragma unroll
                     for (int d = 0; d < DIM; d++) { qa.v[d] = sQ(el, d, na); qb.v[d] = sQ(el, d, nb); }
                     qa.beta = sQ(el, DIM, na); qb.beta = sQ(el, DIM, nb);
@@ -576,7 +485,8 @@ __attribute__((amdgpu_waves_per_eu((LCfg<DIM, NP>::WAVES)))) k_rhs_ln(const KArg
                     qa.lam = sQ(el, DIM + 2, na); qb.lam = sQ(el, DIM + 2, nb);
                     const double si = r == 0 ? A.tab.subn[0][i] : (r == 1 ? A.tab.subn[1][i] : A.tab.subn[2][i]);
                     double G[NV];
-                    ec_flux<DIM, true>(r, si, qa, qb, s1, s2, P, quirk3d, G);
+                    const double ns[3] = {r == 0 ? si : 0.0, r == 1 ? si : 0.0, r == 2 ? si : 0.0};
+                    ec_flux<DIM, true>(ns, si, qa, qb, P, quirk3d, G);
                     const double fa = alpha_e * A.tab.fvs[i];
 #pragma unroll
                     for (int v = 0; v < NV; v++) {
