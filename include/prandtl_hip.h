@@ -287,7 +287,9 @@ int prandtl_set_shape(prandtl_ctx *ctx, int kernel, int shape);
 /* Kernel algorithm of the flux-differencing RHS (no counterpart in the
  * reference; the operator is the same, DGSEMIntegrator.cpp:151-1196).
  * PRANDTL_ALGO_TILE: k_rhs, a workgroup's threads take the element's
- * two-point fluxes as jobs through LDS (every mesh kind).  PRANDTL_ALGO_LINE:
+ * two-point fluxes as jobs through LDS (every mesh kind up to 3-D N = 4; a
+ * context with a single kernel reports this value too, so 3-D boxes of N >= 5,
+ * which run k_rhs_lh, one thread per tensor line).  PRANDTL_ALGO_LINE:
  * k_rhs_ln, one thread per tensor line (periodic Cartesian boxes in 3-D,
  * N = 2..4), the default at N = 2 and 3 and, with blending, at N = 4 (the
  * faster of the two there; unblended N = 4 defaults to the tile kernel);

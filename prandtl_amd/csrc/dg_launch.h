@@ -6,6 +6,7 @@
 #include <vector>
 #include "dg_device.h"
 #include "dg_line.h"
+#include "dg_line_high.h"
 #include "dg_visc_mx.h"
 
 using namespace prandtl;
@@ -213,9 +214,8 @@ inline bool line_default(const prandtl_ctx *c)
 }
 
 template <int DIM, int NP, bool BLEND>
-int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
+int launch_rhs_low(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
-    ProfScope ps(c, s, 0);
     const bool qns3 = DIM == 3 && c->prm.parabolic && c->prm.quirks;
     if constexpr (line_built(DIM, NP)) {
         if (c->rhs_algo == PRANDTL_ALGO_LINE && line_ok(c)) {
@@ -295,6 +295,37 @@ int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
     return hip_check(c, hipGetLastError(), "k_rhs launch");
 }
 
+template <int DIM, int NP, bool BLEND, int FB, bool OPEN>
+void launch_rhs_high(prandtl_ctx *c, const KArgs &a, hipStream_t s)
+{
+    using Hc = HCfg<DIM, NP, FB>;
+    const int nb = (c->NE + Hc::EPB - 1) / Hc::EPB;
+    if (c->prm.parabolic && c->prm.quirks)
+        hipLaunchKernelGGL((k_rhs_lh<DIM, NP, BLEND, true, double, FB, OPEN>), dim3(nb), dim3(Hc::BLOCK), 0, s, a);
+    else if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED)
+        hipLaunchKernelGGL((k_rhs_lh<DIM, NP, BLEND, false, float, FB, OPEN>), dim3(nb), dim3(Hc::BLOCK), 0, s, a);
+    else hipLaunchKernelGGL((k_rhs_lh<DIM, NP, BLEND, false, double, FB, OPEN>), dim3(nb), dim3(Hc::BLOCK), 0, s, a);
+}
+
+template <int DIM, int NP, bool BLEND>
+int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
+{
+    ProfScope ps(c, s, 0);
+    if constexpr (high_built(DIM, NP)) {
+        if (c->geo.bcmask) launch_rhs_high<DIM, NP, BLEND, 0, true>(c, a, s);
+        else {
+            bool done = false;
+            if constexpr (rhs_shape_ok(DIM, NP, BLEND, 3)) {
+                if (c->rhs_shape == 3) {
+                    launch_rhs_high<DIM, NP, BLEND, 256, false>(c, a, s);
+                    done = true;
+                }
+            }
+            if (!done) launch_rhs_high<DIM, NP, BLEND, 0, false>(c, a, s);
+        }
+        return hip_check(c, hipGetLastError(), "k_rhs_lh launch");
+    } else return launch_rhs_low<DIM, NP, BLEND>(c, a, s);
+}
 inline KArgs make_kargs(const prandtl_ctx *c, const double *y, const double *u0, double *out, int mode,
                  double dt, double c0, double c1, const double *dtp)
 {

@@ -119,6 +119,11 @@ __device__ __forceinline__ double atanh_ratio(double u)
     return fma(p, u, 1.0);
 }
 
+// RANGE: LM_ANY chooses per pair; LM_SHORT and LM_MID are the first two alone,
+// for callers that have bounded the ratio of a whole line's values.
+enum { LM_SHORT = 0, LM_MID = 1, LM_ANY = 2 };
+
+template <int RANGE>
 __device__ __forceinline__ void log_means(double ra, double rb, double ba, double bb, double &rho_ln,
                                           double &ibeta_ln, double &rbs)
 {
@@ -127,13 +132,13 @@ __device__ __forceinline__ void log_means(double ra, double rb, double ba, doubl
     rbs = rcp_nr(bs);
     const double fr = dr * rcp_nr(rs), fb = db * rbs;
     const double ur = fr * fr, ub = fb * fb;
-    if ((ur < 1e-4) & (ub < 1e-4)) {
+    if (RANGE == LM_SHORT || (RANGE == LM_ANY && ((ur < 1e-4) & (ub < 1e-4)))) {
         // T = 1 + u/3 + u^2/5 + u^3/7, 1/T = 1 - u/3 - 4u^2/45 - 44u^3/945
         const double tr = fma(ur, fma(ur, fma(ur, -22.0 / 945.0, -2.0 / 45.0), -1.0 / 6.0), 0.5);
         const double tb = fma(ub, fma(ub, fma(ub, 2.0 / 7.0, 2.0 / 5.0), 2.0 / 3.0), 2.0);
         rho_ln = rs * tr;
         ibeta_ln = rbs * tb;
-    } else if ((ur < 1.0 / 9.0) & (ub < 1.0 / 9.0)) {
+    } else if (RANGE == LM_MID || ((ur < 1.0 / 9.0) & (ub < 1.0 / 9.0))) {
         rho_ln = 0.5 * rs * rcp_nr(atanh_ratio(ur));
         ibeta_ln = 2.0 * rbs * atanh_ratio(ub);
     } else {
@@ -153,12 +158,12 @@ __device__ __forceinline__ void log_means(double ra, double rb, double ba, doubl
 //  - the momentum jump is rho_mean dv + drho v_mean, and the energy jump
 //    reuses drho h, so the conserved states are not read.
 // Symmetric in (a, b) for DISS = false, as the symmetric pairs need.
-template <int DIM, bool DISS>
+template <int DIM, bool DISS, int RANGE = LM_ANY>
 __device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<DIM> &a, const NodeQ<DIM> &b,
                                         const Phys &P, bool quirk3d, double *F)
 {
     double rho_ln, ibeta_ln, rbs;
-    log_means(a.rho, b.rho, a.beta, b.beta, rho_ln, ibeta_ln, rbs);
+    log_means<RANGE>(a.rho, b.rho, a.beta, b.beta, rho_ln, ibeta_ln, rbs);
     double vs[DIM];
     double h2 = 0.0, w = 0.0;
 #pragma unroll
@@ -193,99 +198,6 @@ __device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<
             else e = fma(dv, vs[d], e);
         }
         F[DIM + 1] = fma(-hl, fma(drho, h, fma(0.5 * rm, e, q3)), F[DIM + 1]);
-    }
-}
-
-// The division form of the two-point flux, which the 3-D tile kernel keeps at
-// N >= 5: its 128-register build spills with ec_flux's three ranges (3-D N =
-// 7 with blending, 32^3: 3.46 ms per right-hand side with this form, 4.28 with
-// ec_flux).
-// Logarithmic mean LM(x,y) and its reciprocal, ComputeLogMean of
-// BasicOperations.cpp:6-12 (eps = 1e-4).  With d = y-x, s = y+x the
-// reference's u = ((xi-1)/(xi+1))^2 with xi = y/x is d^2/s^2, so the branch
-// test u < eps is q < eps*t (q = d^2, t = s^2) and the series branch
-//   LM = 52.5 s / (105 + 35u + 21u^2 + 15u^3)
-//      = 52.5 s t^3 / (((15 q + 21 t) q + 35 t^2) q + 105 t^3)
-// costs one division instead of three.  The log branch keeps the reference's
-// (y-x)/log(y/x).  Either form differs from the reference's by rounding only
-// (t^3 stays in range for |x|,|y| in 1e-40..1e40).
-__device__ __forceinline__ double lm_series_den(double q, double t)
-{
-    return ((15.0 * q + 21.0 * t) * q + 35.0 * t * t) * q + 105.0 * t * t * t;
-}
-
-__device__ __forceinline__ double logmean(double x, double y)
-{
-    const double d = y - x, s = y + x;
-    const double q = d * d, t = s * s;
-    if (q < 1e-4 * t) return 52.5 * s * (t * t * t) / lm_series_den(q, t);
-    return d / log(y / x);
-}
-
-__device__ __forceinline__ double inv_logmean(double x, double y)
-{
-    const double d = y - x, s = y + x;
-    const double q = d * d, t = s * s;
-    if (q < 1e-4 * t) return lm_series_den(q, t) / (52.5 * s * (t * t * t));
-    return log(y / x) / d;
-}
-
-// Chandrashekar two-point flux for the normal nr e_r (nr signed) whose
-// dissipation is scaled by nd = |nr| (the face normal's Norml2,
-// ChandrashekarFlux.cpp:88).  DISS = false: ComputeVolumeFlux
-// (ChandrashekarFlux.cpp:11-83), metric mean of two equal metrics.
-// DISS = true: ComputeFaceFlux (lines 85-161) with the conserved states s1,
-// s2 for the jumps; quirk3d keeps the 3-D energy dissipation term of line
-// 131.  Only 1/beta_ln enters the fluxes, so the beta log mean is formed as
-// its reciprocal.
-template <int DIM, bool DISS>
-__device__ __forceinline__ void two_point_flux(int r, double nr, double nd, const NodeQ<DIM> &a,
-                                               const NodeQ<DIM> &b, const double *s1,
-                                               const double *s2, const Phys &P, bool quirk3d,
-                                               double *F)
-{
-    const double rho_ln = logmean(a.rho, b.rho);
-    const double rho_mean = 0.5 * (a.rho + b.rho);
-    const double drho = b.rho - a.rho;
-    double vm[DIM];
-    double h_hat = 0.0, diss = 0.0;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        vm[d] = 0.5 * (a.v[d] + b.v[d]);
-        const double hd = -0.25 * (a.v[d] * a.v[d] + b.v[d] * b.v[d]) + vm[d] * vm[d];
-        h_hat = (d == 0) ? hd : h_hat + hd;
-        if (DISS) {
-            const double dv = b.v[d] - a.v[d];
-            const double t0 = 0.5 * drho * a.v[d] * b.v[d];
-            const double dd = (DIM == 3 && d == 2 && quirk3d) ? t0 + rho_mean * dv + vm[d]
-                                                              : t0 + rho_mean * dv * vm[d];
-            diss = (d == 0) ? dd : diss + dd;
-        }
-    }
-    double vr = vm[0];
-#pragma unroll
-    for (int d = 1; d < DIM; d++)
-        if (d == r) vr = vm[d];
-    const double Vn = vr * nr;
-    const double ibeta_ln = inv_logmean(a.beta, b.beta);
-    const double p_hat = 0.5 * (a.rho + b.rho) / (a.beta + b.beta);
-    h_hat += 0.5 * ibeta_ln * P.gm1i + p_hat / rho_ln;
-    const double rVn = rho_ln * Vn;
-    F[0] = rVn;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        const double mom = rho_ln * vm[d];
-        F[1 + d] = (d == r) ? Vn * mom + p_hat * nr : Vn * mom;
-    }
-    F[DIM + 1] = rVn * h_hat;
-    if (DISS) {
-        diss += 0.5 * drho * P.gm1i * ibeta_ln + 0.5 * rho_mean * P.gm1i * (b.ibeta - a.ibeta);
-        const double lam = (a.lam < b.lam) ? b.lam : a.lam;
-        const double hl = 0.5 * lam;
-        F[0] = F[0] - hl * (s2[0] - s1[0]) * nd;
-#pragma unroll
-        for (int d = 0; d < DIM; d++) F[1 + d] = F[1 + d] - hl * (s2[1 + d] - s1[1 + d]) * nd;
-        F[DIM + 1] = F[DIM + 1] - hl * diss * nd;
     }
 }
 
