@@ -285,20 +285,15 @@ int prandtl_set_graph(prandtl_ctx *ctx, int enable);
 int prandtl_set_shape(prandtl_ctx *ctx, int kernel, int shape);
 
 /* Kernel algorithm of the flux-differencing RHS (no counterpart in the
- * reference; the operator is the same, DGSEMIntegrator.cpp:151-1196).
- * PRANDTL_ALGO_TILE: k_rhs, a workgroup's threads take the element's
- * two-point fluxes as jobs through LDS (every mesh kind up to 3-D N = 4; a
- * context with a single kernel reports this value too, so 3-D boxes of N >= 5,
- * which run k_rhs_lh, one thread per tensor line).  PRANDTL_ALGO_LINE:
- * k_rhs_ln, one thread per tensor line (periodic Cartesian boxes in 3-D,
- * N = 2..4), the default at N = 2 and 3 and, with blending, at N = 4 (the
- * faster of the two there; unblended N = 4 defaults to the tile kernel);
- * with it, the mixed form at N = 3
- * runs its viscous kernel's derivative contractions on the FP32 matrix cores
- * (k_visc_mx).  The two differ by rounding only;
- * launch shapes (prandtl_set_shape, prandtl_autotune) belong to the current
- * algorithm (the line kernel has shape 0 only).  PRANDTL_ERR_UNSUPPORTED for
- * an algorithm this case does not have. */
+ * reference; the operator is the same, DGSEMIntegrator.cpp:151-1196).  Every
+ * 2-D and 3-D mesh runs k_rhs_l, one thread per tensor line.  Periodic
+ * Cartesian boxes in 3-D, N = 2..4, have two settings: PRANDTL_ALGO_LINE (the
+ * default at N = 2 and 3 and, with blending, at N = 4) runs the mixed form's
+ * viscous kernel at N = 3 with its derivative contractions on the FP32
+ * matrix cores (k_visc_mx) and has launch shape 0 only; PRANDTL_ALGO_TILE
+ * runs k_visc and has the forced launch shapes.  Their FP64 results are the
+ * same.  Every other context reports PRANDTL_ALGO_TILE, and
+ * PRANDTL_ERR_UNSUPPORTED for PRANDTL_ALGO_LINE. */
 #define PRANDTL_ALGO_TILE 0
 #define PRANDTL_ALGO_LINE 1
 int prandtl_set_algorithm(prandtl_ctx *ctx, int kernel, int algo);
@@ -439,8 +434,8 @@ const char *prandtl_ensemble_last_error(const prandtl_ensemble *ens);
 
 /* Launch form of the ensemble's stages (no counterpart in the reference):
  * mode 0 launches one workgroup per element tile (the cost-sorted tile list
- * is the dispatch order); mode g = 1..PRANDTL_ENS_MAX_PER_CU launches g
- * persistent workgroups per CU that take tiles from a device counter until
+ * is the dispatch order); mode g = 1..PRANDTL_ENS_MAX_PER_CU launches 4 g
+ * persistent workgroups of one wave per CU that take tiles from a device counter until
  * the list is exhausted.  Every form gives bitwise the same results. */
 #define PRANDTL_ENS_MAX_PER_CU 4
 int prandtl_ensemble_set_mode(prandtl_ensemble *ens, int mode);

@@ -1,6 +1,7 @@
-// Device side of the DGSEM RHS (gfx950): tables, launch shapes, the k_rhs
-// tile body and the k_rhs / k_visc kernel templates.  Included by the
-// library's host translation unit and by the per-order instantiation units.
+// Device side of the DGSEM RHS (gfx950): tables and arguments, launch shapes,
+// mesh and index helpers, the 1-D kernel k_rhs and the viscous kernel k_visc.
+// Included by the library's host translation unit and by the per-order
+// instantiation units.
 //
 // Two kernels per RHS evaluation:
 //
@@ -12,28 +13,14 @@
 //      node).  Restates DGSEMOperator.cpp:82-159, LiftingBR1.cpp:10-272 and
 //      DGSEMIntegrator.cpp:617-641,705-738 (and 435-549 for the face side).
 //
-//  k_rhs  the inviscid flux differencing, surface fluxes, modal indicator and
-//      subcell FV blending, plus the viscous volume/face terms from k_visc,
-//      then either writes the RHS (Operator::Mult) or the RK3 stage
-//      combination.  Restates DGSEMIntegrator.cpp:151-433,435-549,601-864,
-//      972-1196, PerssonPeraireIndicator.cpp:21-58, DGSEMOperator.cpp:60-80
-//      and MFEM's RK3SSPSolver stage arithmetic.
+//  k_rhs_l (dg_lines.h; k_rhs in 1-D)  the inviscid flux differencing,
+//      surface fluxes, modal indicator and subcell FV blending, plus the
+//      viscous volume/face terms from k_visc, then either writes the RHS
+//      (Operator::Mult) or the RK3 stage combination.
 //
-// Work decomposition: a workgroup owns EPB whole elements (one node per
-// thread in the node phases).  For each direction the element's two-point
-// fluxes are "jobs" — symmetric volume pairs (computed once, as the
-// reference does), surface points and subcell interfaces — computed by all
-// threads into LDS, then reduced per node in the reference's summation
-// order.  Face jobs are computed by both neighbouring elements ("owner
-// computes") with the face's canonical orientation, so each face point's flux
-// is bitwise the same on both sides and no atomics or scatter are needed.
-// k_rhs is instantiated for DIM = 1, 2 and 3 (1-D: one line per element, a
-// single point per face, unit face normals; Euler only, so no k_visc).
-//
-// Both kernels are also built for forced workgroup sizes (64, 128 or 256
-// threads, "launch shapes"); prandtl_autotune picks one per context by
-// timing them on the caller's state.  k_ens runs k_rhs's tile body over the
-// element tiles of many independent 2-D cases in one launch per RK stage.
+// Both are also built for forced workgroup sizes (64, 128 or 256 threads,
+// "launch shapes"); prandtl_autotune picks one per context by timing them on
+// the caller's state.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -335,18 +322,10 @@ __device__ __forceinline__ void block_lam_max(double lam, double old, double *sl
     }
 }
 
-// ---------------------------------------------------------------------------
-// k_rhs
-// ---------------------------------------------------------------------------
-// Launch shape of k_rhs: per element the work items are K nodes, JF surface
-// points (all 2*DIM faces) and, per direction, JP volume pairs plus JV
-// subcell interfaces.  EPB elements per workgroup are chosen so that each
-// phase gives every thread about one item (3-D N=3: 2 elements, 192
-// threads: 96 surface points and 96 pairs per direction per element).
-//
-// FB (forced block size, 0 = natural) gives the other launch shapes the
-// autotuner tries; rshape() computes a shape without instantiating RCfg, so
-// the host can test which shapes exist.
+// Launch shapes of the RHS in two and three dimensions: which workgroup sizes
+// a caller may force (PRANDTL_SHAPES).  A shape is offered where a workgroup
+// of its size holds an element's nodes one per thread and differs from the
+// size rshape() gives as the natural one.
 struct RShape {
     int K, WORK, EPB, BLOCK;
 };
@@ -360,8 +339,6 @@ constexpr RShape rshape(int DIM, int NP, bool BLEND, int FB)
     const int BLOCK = FB ? FB : K > 256 ? r64(K) : (r64(EPB * WORK) > 512 ? 512 : r64(EPB * WORK));
     return RShape{K, WORK, EPB, BLOCK};
 }
-// A forced k_rhs shape exists when it holds one node per thread and differs
-// from the natural one.
 constexpr bool rhs_shape_ok(int DIM, int NP, bool BLEND, int shape)
 {
     if (shape == 0) return true;
@@ -370,56 +347,6 @@ constexpr bool rhs_shape_ok(int DIM, int NP, bool BLEND, int shape)
     const RShape f = rshape(DIM, NP, BLEND, shape_fb(shape));
     return f.EPB * f.K <= f.BLOCK && !(f.EPB == n.EPB && f.BLOCK == n.BLOCK);
 }
-
-template <int DIM, int NP, bool BLEND, int FB = 0> struct RCfg {
-    static constexpr int NV = DIM + 2;
-    static constexpr int K = npow(NP, DIM);
-    static constexpr int NFP = npow(NP, DIM - 1);
-    static constexpr int NPAIR = NP * (NP - 1) / 2;
-    static constexpr int NFV = BLEND ? NP - 1 : 0;
-    static constexpr int JP = NFP * (NPAIR + NFV);
-    static constexpr int JF = 2 * DIM * NFP;
-    static constexpr int WORK = rshape(DIM, NP, BLEND, FB).WORK;
-    static constexpr int EPB = rshape(DIM, NP, BLEND, FB).EPB;
-    static constexpr int BLOCK = rshape(DIM, NP, BLEND, FB).BLOCK;
-    static constexpr int lc_pick()
-    {
-        for (int lc = NFP; lc >= 1; lc--)
-            if (NFP % lc == 0 && EPB * lc * (NPAIR + NFV) * NV * 8 <= 32 * 1024) return lc;
-        return 1;
-    }
-    static constexpr int LC = lc_pick();
-    static constexpr int FXN = LC * (NPAIR + NFV);
-    // registers for 4 waves per SIMD (128) where a workgroup has at most two
-    // waves, otherwise PRANDTL_WAVES
-    static constexpr int WAVES = BLOCK <= 128 ? 4 : PRANDTL_WAVES;
-    static_assert(EPB * K <= BLOCK, "one node per thread");
-};
-
-// LDS of one k_rhs tile (EPB elements).
-template <int DIM, int NP, bool BLEND, bool QNS3, int FB, bool GEN = false, bool AXI = false> struct RhsSmem {
-    using C = RCfg<DIM, NP, BLEND, FB>;
-    static constexpr int NQ = DIM + 1 + (BLEND ? 2 : 0);   // v[DIM], beta, (1/beta, lambda)
-    static constexpr int GK = QNS3 ? C::K : 1, GE = QNS3 ? C::EPB : 1;
-    double Dh2[NP * NP];
-    double V1i[BLEND ? NP * NP : 1];
-    double Fvs[NP];
-    double Sub[DIM][NP];
-    double U[C::EPB][C::NV][C::K];
-    double Q[C::EPB][NQ][C::K];
-    // signed surface contributions (surface phase), then the pair and
-    // subcell fluxes of one line chunk (direction phases): one buffer
-    // (also the indicator's scratch: 4 K values per element)
-    static constexpr int FF = cmx(cmx(C::JF, C::FXN), BLEND ? (4 * C::K + C::NV - 1) / C::NV : 1);
-    static_assert(!BLEND || 4 * C::K <= C::NV * FF, "indicator scratch fits the flux buffer");
-    double F[C::EPB][C::NV][FF];
-    double G[GE][C::NV][GK];
-    double Al[C::EPB];
-    double Red[(C::BLOCK + 63) / 64];
-    double M[GEN ? C::EPB : 1][GEN ? DIM * DIM : 1][GEN ? C::K : 1];   // per-node adjugate rows (general geometry)
-    double R[AXI ? C::EPB : 1][AXI ? C::K : 1];      // per-node r (axisymmetric)
-    double Cn[GEN && DIM == 3 ? C::EPB : 1][GEN && DIM == 3 ? 24 : 1];   // hexahedron corners
-};
 
 // DGSEMOperator::RecoverStateFromWeighted (DGSEMOperator.cpp:161-424) for one
 // node q: U = rU / r off the axis; on it (low-order axis reconstruction, as
@@ -531,234 +458,122 @@ template <int NP> __device__ __forceinline__ int face_point_3(int node, int r)
     return r == 0 ? j + NP * k : (r == 1 ? i + NP * k : i + NP * j);
 }
 
-// One tile of k_rhs: elements [tile*EPB, tile*EPB + EPB) of the case A
-// describes; slot indexes the tile's running wave-speed maximum.
-// BLEND: modal indicator + subcell FV blending compiled in.
-// QNS3: the reference's NS-3D zeta-partner defect (faithful NS in 3-D).
-// VT: element type of the viscous inputs from k_visc (float in the mixed form).
-// FB: forced workgroup size (0: the natural one of RCfg).
-// OPEN: boundary sides on a Cartesian box.  GEN: general geometry of a
-// quadrilateral or hexahedral mesh (per-node metrics, face tables; boundaries
-// by attribute).  AXI
-// (with GEN, Euler): axisymmetric, A.y the weighted state r U, recovered
-// node by node as it is loaded (this element's nodes and the neighbours'
-// face points); two-point, subcell and face fluxes weighted by r, the radial
-// momentum's pressure source, its RHS zeroed on the axis.
-template <int DIM, int NP, bool BLEND, bool QNS3, typename VT, int FB, bool OPEN = false, bool GEN = false,
-          bool AXI = false>
-__device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const int slot,
-                                         RhsSmem<DIM, NP, BLEND, QNS3, FB, GEN, AXI> &S, const int tid = -1)
+// ---------------------------------------------------------------------------
+// k_rhs: 1-D boxes (Euler)
+// ---------------------------------------------------------------------------
+// A workgroup's threads take the elements' two-point fluxes as jobs: one node
+// per thread in the node phases, then surface points, then symmetric volume
+// pairs and subcell interfaces through LDS, summed per node in the
+// reference's order.  A 1-D mesh has one line per element, so a thread per
+// line (k_rhs_l) would leave a mesh of a few hundred elements with a handful of
+// waves and all of a line's fluxes in sequence: 128 elements with a shock, 32
+// steps of the device loop 1,560 us against 1,130 here.
+template <int NP, bool BLEND> struct R1Cfg {
+    static constexpr int NPAIR = NP * (NP - 1) / 2;
+    static constexpr int NFV = BLEND ? NP - 1 : 0;
+    static constexpr int JOBS = NPAIR + NFV;
+    static constexpr int WORK = cmx(NP, cmx(JOBS, 2));
+    static constexpr int EPB = cmx(1, 256 / WORK);
+    static constexpr int BLOCK = r64(EPB * WORK) > 512 ? 512 : r64(EPB * WORK);
+    static_assert(EPB * NP <= BLOCK, "one node per thread");
+};
+
+template <int NP, bool BLEND, bool OPEN>
+__global__ void __launch_bounds__((R1Cfg<NP, BLEND>::BLOCK))
+__attribute__((amdgpu_waves_per_eu(3))) k_rhs(const KArgs A)
 {
-    using C = RCfg<DIM, NP, BLEND, FB>;
-    constexpr int NV = C::NV, K = C::K, NFP = C::NFP, NPAIR = C::NPAIR, NFV = C::NFV;
-    constexpr int EPB = C::EPB, LC = C::LC, BLOCK = C::BLOCK, FXN = C::FXN, JF = C::JF;
-    constexpr int NQ = RhsSmem<DIM, NP, BLEND, QNS3, FB, GEN, AXI>::NQ;
-    static_assert(!AXI || (GEN && DIM == 2), "axisymmetric meshes are quadrilateral meshes");
-    constexpr int MC = DIM * DIM;   // adjugate entries per node (general geometry)
-    auto &sM = S.M;
-    (void)sM;
-    auto &sR = S.R;
-    (void)sR;
-    (void)FXN;
-    auto &sDh2 = S.Dh2;
-    auto &sV1i = S.V1i;
-    auto &sFvs = S.Fvs;
-    auto &sSub = S.Sub;
-    auto &sU = S.U;
-    auto &sQ = S.Q;
-    auto &sF = S.F;
-    auto &sFc = S.F;
-    auto &sG = S.G;
-    auto &sAl = S.Al;
-    auto &sRed = S.Red;
+    using C = R1Cfg<NP, BLEND>;
+    constexpr int NV = 3, NPAIR = C::NPAIR, NFV = C::NFV, JOBS = C::JOBS, EPB = C::EPB, BLOCK = C::BLOCK;
+    constexpr int NQ = BLEND ? 4 : 2;   // v, beta, (1/beta, lambda)
+    constexpr int FF = cmx(cmx(JOBS, 2), BLEND ? (4 * NP + NV - 1) / NV : 1);
+    static_assert(!BLEND || 4 * NP <= NV * FF, "indicator scratch fits the flux buffer");
+    __shared__ double sDh2[NP * NP], sV1i[BLEND ? NP * NP : 1], sFvs[NP], sSub[NP];
+    __shared__ double sU[EPB][NV][NP], sQ[EPB][NQ][NP];
+    __shared__ double sF[EPB][NV][FF];   // surface contributions, then the pair and subcell fluxes
+    __shared__ double sAl[EPB], sRed[(BLOCK + 63) / 64];
 
     if (A.skip && *A.skip) return;   // uniform: before any barrier
-    // tid: the thread's index as the caller sees it (a loop over tiles passes
-    // one the compiler cannot hoist out of the loop)
-    const int t = tid < 0 ? (int)threadIdx.x : tid;
+    const int t = threadIdx.x;
     // the operator's tables, one entry per thread, loaded together and first
     // (indices clamped, so every lane loads and no load waits for another);
     // they go to LDS once the prologue's loads are in flight
     static_assert(NP * NP <= BLOCK, "one table entry per thread");
-    const int tq = t < NP * NP ? t : 0, tf = t < NP ? t : 0, ts = t < DIM * NP ? t : 0;
+    const int tq = t < NP * NP ? t : 0, tf = t < NP ? t : 0;
     const double tDh2 = A.tab.Dh2[(tq / NP) * MAXNP + tq % NP];
     const double tV1i = BLEND ? A.tab.V1i[(tq / NP) * MAXNP + tq % NP] : 0.0;
-    const double tFvs = A.tab.fvs[tf];
-    const double tSub = A.tab.subn[ts / NP][ts % NP];
+    const double tFvs = A.tab.fvs[tf], tSub = A.tab.subn[0][tf];
 
     const Phys &P = A.phys;
     const int NE = A.geo.NE;
-    const size_t NK = (size_t)NE * K;
+    const size_t NK = (size_t)NE * NP;
+    const int tile = xcd_remap(blockIdx.x, gridDim.x);
     const int ebase = tile * EPB;
-    const int el = t / K;
-    const int n = t - el * K;
+    const int el = t / NP, n = t - el * NP;
     const int e = ebase + el;
     const bool act = (el < EPB) && (e < NE);
-    const bool quirk3d = A.quirks != 0;
-    const int ii[3] = {n % NP, (n / NP) % NP, DIM == 3 ? n / (NP * NP) : 0};
-
-    // ---- prologue: own node state, the neighbour data of this thread's
-    // first surface point, the step size and the tile's wave-speed slot, all
-    // loads in flight together ----
     const double dt = step_dt(A);
-    const double lam_old = (t == 0) ? A.lam[slot] : 0.0;
+    const double lam_old = (t == 0) ? A.lam[blockIdx.x] : 0.0;
     double ys[NV];
     if (act)
 #pragma unroll
-        for (int v = 0; v < NV; v++) ys[v] = A.y[v * NK + (size_t)e * K + n];
-    // general geometry: this node's adjugate rows and Jacobian (and r)
-    double jn = 1.0, mown[GEN ? MC : 1], rown = 0.0;
-    int axown = -1;
-    double yw[AXI ? NV : 1];   // axisymmetric: the weighted state of the update
-#pragma unroll
-    for (int c = 0; c < (GEN ? MC : 1); c++) mown[c] = 0.0;
-    if (AXI && act) {
-        rown = A.geo.rnode[(size_t)e * K + n];
-        axown = A.geo.axm[(size_t)e * K + n];
-#pragma unroll
-        for (int v = 0; v < NV; v++) yw[v] = ys[v];
-        axis_node(A.y, A.geo, K, NK, (size_t)e * K + n, ys);
-    }
-    if constexpr (GEN && DIM == 3) {
-        // the tile's corners into LDS, then each node's metrics from them
-        for (int i = t; i < EPB * 24; i += BLOCK)
-            S.Cn[i / 24][i % 24] = (ebase + i / 24 < NE) ? A.geo.corner[(size_t)(ebase + i / 24) * 24 + i % 24] : 0.0;
-        __syncthreads();
-        if (act) hex_metrics(S.Cn[el], A.tab.x[ii[0]], A.tab.x[ii[1]], A.tab.x[ii[2]], mown, jn);
-    } else if constexpr (GEN) {
-        if (act) {
-            jn = A.geo.jac[(size_t)e * K + n];
-#pragma unroll
-            for (int c = 0; c < MC; c++) mown[c] = A.geo.met[c * NK + (size_t)e * K + n];
-        }
-    }
-    // Blended kernels carry the subcell-flux work and its accumulator; they
-    // do not hold loads in flight across phases (the surface data is loaded
-    // in the surface phase, the assembly inputs at the assembly), which keeps
-    // their register count down.
-    constexpr bool PREFETCH = !BLEND && !GEN;
-    double pn[NV], pfo[NV], pfn[NV];
-    if constexpr (PREFETCH) {
-        const int jf = t;
-        const int ej = jf / JF;
-        const int eo = ebase + ej;
-        if (jf < EPB * JF && eo < NE) {
-            const int rem = jf - ej * JF;
-            const int f = rem / NFP, l = rem - f * NFP;
-            const int r = f >> 1, side = f & 1;
-            const int en = neighbor_lane(A.geo, eo, r, side);
-            const int nn = line_node<DIM, NP>(r, l, side ? 0 : NP - 1);
-#pragma unroll
-            for (int v = 0; v < NV; v++) pn[v] = A.y[v * NK + (size_t)en * K + nn];
-            if (A.parabolic) {
-                const VT *fo = static_cast<const VT *>(A.fvf) + (((size_t)eo * 2 * DIM + f) * (NV - 1)) * NFP;
-                const VT *fn = static_cast<const VT *>(A.fvf) + (((size_t)en * 2 * DIM + (f ^ 1)) * (NV - 1)) * NFP;
-#pragma unroll
-                for (int v = 1; v < NV; v++) { pfo[v] = fo[(v - 1) * NFP + l]; pfn[v] = fn[(v - 1) * NFP + l]; }
-            }
-        }
-    }
-
+        for (int v = 0; v < NV; v++) ys[v] = A.y[v * NK + (size_t)e * NP + n];
     if (t < NP * NP) {
         sDh2[t] = tDh2;
         if (BLEND) sV1i[t] = tV1i;
     }
-    if (t < NP) sFvs[t] = tFvs;
-    if (t < DIM * NP) sSub[t / NP][t % NP] = tSub;
+    if (t < NP) { sFvs[t] = tFvs; sSub[t] = tSub; }
 
     // ---- node phase: state and per-node flux quantities into LDS ----
     double lam = 0.0;
     if (act) {
 #pragma unroll
         for (int v = 0; v < NV; v++) sU[el][v][n] = ys[v];
-        if constexpr (GEN)
-#pragma unroll
-            for (int c = 0; c < MC; c++) sM[el][c][n] = mown[c];
-        if constexpr (AXI) sR[el][n] = rown;
-        const NodeQ<DIM> q = node_quants<DIM>(ys, P);
-#pragma unroll
-        for (int d = 0; d < DIM; d++) sQ[el][d][n] = q.v[d];
-        sQ[el][DIM][n] = q.beta;
+        const NodeQ<1> q = node_quants<1>(ys, P);
+        sQ[el][0][n] = q.v[0];
+        sQ[el][1][n] = q.beta;
         if constexpr (BLEND) {
-            sQ[el][DIM + 1][n] = q.ibeta;
-            sQ[el][DIM + 2][n] = q.lam;
+            sQ[el][2][n] = q.ibeta;
+            sQ[el][3][n] = q.lam;
         }
         lam = (q.lam == q.lam) ? q.lam : 0.0;
-        if (QNS3 && ii[1] == NP - 1)
-#pragma unroll
-            for (int v = 0; v < NV; v++) sG[el][v][n] = 0.0;
     }
     __syncthreads();
 
     // ---- modal indicator and blending coefficient (element-local) ----
-    if (BLEND) {
+    if constexpr (BLEND) {
         double *sX = &sF[0][0][0];
-        double *sY = sX + EPB * K;
+        double *sM = sX + EPB * NP, *sE1 = sX + 2 * EPB * NP, *sE2 = sX + 3 * EPB * NP;
         if (act) {
             // rho * ComputePressure(state) with V /= rho (BasicOperations.cpp:31-37)
-            const double rr = 1.0 / ys[0];
-            double vv = 0.0;
-#pragma unroll
-            for (int d = 0; d < DIM; d++) {
-                const double v = ys[1 + d] * rr;
-                vv = (d == 0) ? v * v : vv + v * v;
-            }
-            sX[el * K + n] = ys[0] * (P.gm1 * (ys[DIM + 1] - 0.5 * ys[0] * vv));
+            const double v = ys[1] * (1.0 / ys[0]);
+            sX[el * NP + n] = ys[0] * (P.gm1 * (ys[2] - 0.5 * ys[0] * (v * v)));
         }
         __syncthreads();
-        // modes = V^-1 q, V^-1 = kron of the 1-D inverses, one direction at a time
-        double *src = sX, *dst = sY;
-#pragma unroll
-        for (int r = 0; r < DIM; r++) {
-            if (act) {
-                const int a = ii[r];
-                double s = 0.0;
-#pragma unroll
-                for (int i = 0; i < NP; i++) {
-                    int jj[3] = {ii[0], ii[1], ii[2]};
-                    jj[r] = i;
-                    const int m = DIM == 2 ? jj[1] * NP + jj[0] : (jj[2] * NP + jj[1]) * NP + jj[0];
-                    s = (i == 0) ? sV1i[a * NP + i] * src[el * K + m] : s + sV1i[a * NP + i] * src[el * K + m];
-                }
-                dst[el * K + n] = s;
-            }
-            __syncthreads();
-            double *tmp = src; src = dst; dst = tmp;
-        }
-        // modal energies: all modes, modes of degree <= N-1 and <= N-2 in
-        // every direction (masks of PerssonPeraireIndicator.cpp:38-52).  Node
-        // n holds the mode of degrees ii[] (mode order of ModalBasis.cpp:72-104
-        // maps to this position); the three sums are a binary tree over the
-        // element's K entries, the same for every launch shape.
-        double *sE0 = dst, *sE1 = sX + 2 * EPB * K, *sE2 = sX + 3 * EPB * K;
         if (act) {
-            const double md = src[el * K + n];
-            bool in1 = true, in2 = true;
+            double s = 0.0;
 #pragma unroll
-            for (int d = 0; d < DIM; d++) {
-                if (ii[d] > NP - 3) in2 = false;
-                if (ii[d] > NP - 2) in1 = false;
-            }
-            const double e2 = md * md;
-            sE0[el * K + n] = e2;
-            sE1[el * K + n] = in1 ? e2 : 0.0;
-            sE2[el * K + n] = in2 ? e2 : 0.0;
+            for (int i = 0; i < NP; i++)
+                s = (i == 0) ? sV1i[n * NP + i] * sX[el * NP + i] : s + sV1i[n * NP + i] * sX[el * NP + i];
+            // modal energies: all modes, modes of degree <= N-1 and <= N-2
+            // (PerssonPeraireIndicator.cpp:38-52), summed by a binary tree
+            const double e2 = s * s;
+            sM[el * NP + n] = e2;
+            sE1[el * NP + n] = n <= NP - 2 ? e2 : 0.0;
+            sE2[el * NP + n] = n <= NP - 3 ? e2 : 0.0;
         }
         __syncthreads();
-        constexpr int HALF = pow2_at_least(K) / 2;
 #pragma unroll
-        for (int h = HALF; h >= 1; h >>= 1) {
-            if (act && n < h && n + h < K) {
-                const int i0 = el * K + n;
-                sE0[i0] += sE0[i0 + h];
+        for (int h = pow2_at_least(NP) / 2; h >= 1; h >>= 1) {
+            if (act && n < h && n + h < NP) {
+                const int i0 = el * NP + n;
+                sM[i0] += sM[i0 + h];
                 sE1[i0] += sE1[i0 + h];
                 sE2[i0] += sE2[i0 + h];
             }
             __syncthreads();
         }
-        double mm = 0.0, m1 = 0.0, m2 = 0.0;
-        if (act && n == 0) { mm = sE0[el * K]; m1 = sE1[el * K]; m2 = sE2[el * K]; }
         if (act && n == 0) {
+            const double mm = sM[el * NP], m1 = sE1[el * NP], m2 = sE2[el * NP];
             double eta = 1.0 - m1 / mm;
             const double eta2 = 1.0 - m2 / m1;
             eta = (eta < eta2) ? eta2 : eta;
@@ -775,200 +590,35 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
     }
     const double alpha_e = (BLEND && act) ? sAl[el] : 0.0;
 
-    // ---- surface points of all faces (canonical orientation: elem1 = low
-    // side, normal +e_r), signed contribution for this element ----
-    for (int jf = t; jf < EPB * JF; jf += BLOCK) {
-        const int ej = jf / JF;
+    // ---- the element's two surface points (elem1 = low side, normal +e_x),
+    // signed contribution for this element ----
+    const double nr = A.geo.nrm[0];
+    for (int jf = t; jf < EPB * 2; jf += BLOCK) {
+        const int ej = jf >> 1, side = jf & 1;
         const int eo = ebase + ej;
         if (eo >= NE) continue;
-        const int rem = jf - ej * JF;
-        const int f = rem / NFP, l = rem - f * NFP;
-        const int r = f >> 1, side = f & 1;
-        const double nr = lane_pick3(A.geo.nrm[0], A.geo.nrm[1], A.geo.nrm[2], r);
-        if (!GEN && (!PREFETCH || jf != t)) {
-            // not prefetched, or more surface points than threads: load now
-            const int en = neighbor_lane(A.geo, eo, r, side);
-            const int nn = line_node<DIM, NP>(r, l, side ? 0 : NP - 1);
+        const int no = side ? NP - 1 : 0;
+        const int en = neighbor_lane(A.geo, eo, 0, side);
+        double so[NV], pn[NV], F[NV];
 #pragma unroll
-            for (int v = 0; v < NV; v++) pn[v] = A.y[v * NK + (size_t)en * K + nn];
-            if (A.parabolic) {
-                const VT *fo = static_cast<const VT *>(A.fvf) + (((size_t)eo * 2 * DIM + f) * (NV - 1)) * NFP;
-                const VT *fn = static_cast<const VT *>(A.fvf) + (((size_t)en * 2 * DIM + (f ^ 1)) * (NV - 1)) * NFP;
-#pragma unroll
-                for (int v = 1; v < NV; v++) { pfo[v] = fo[(v - 1) * NFP + l]; pfn[v] = fn[(v - 1) * NFP + l]; }
-            }
-        }
-        const int no = line_node<DIM, NP>(r, l, side ? NP - 1 : 0);
-        double so[NV];
-#pragma unroll
-        for (int v = 0; v < NV; v++) so[v] = sU[ej][v][no];
-        if constexpr (GEN) {
-            // general geometry: the face's normal and first element from the
-            // face tables (owner computes, as on the box), boundary points by
-            // attribute
-            const size_t efo = (size_t)eo * (2 * DIM) + f;
-            const int code = A.geo.fface[efo];
-            const int bt = (code >> 1) & 7;
-            double nvec[DIM];
-#pragma unroll
-            for (int d = 0; d < DIM; d++) nvec[d] = A.geo.fnor[(efo * NFP + l) * DIM + d];
-            // viscous traces Fv.n (the face's normal) of this side, and of the
-            // neighbour's matching point
-            const VT *fvfp = static_cast<const VT *>(A.fvf);
-            double F[NV];
-            if (bt != BC_PERIODIC) {
-                // the attribute's outer state, copied (a pointer that could
-                // aim at either this array or the table would keep the
-                // array in scratch memory)
-                double bs[5];
-#pragma unroll
-                for (int v = 0; v < 5; v++) bs[v] = A.geo.bcs[(code >> 4) * 5 + v];
-                if (A.geo.bfn && A.geo.bfn[(code >> 4) * 16] != 0.0) {
-                    // the attribute's time-dependent outer state at this
-                    // point: "below" where n . x - offset - speed t < 0
-                    // (SpecifiedStateBdrFaceIntegrator.cpp:24-34), evaluated
-                    // left to right without contraction
-                    const double *fn = A.geo.bfn + (code >> 4) * 16;
-                    const double *xp = A.geo.fxy + (efo * NFP + l) * 2;
-                    const double tt = (A.tp ? *A.tp : 0.0) + A.tc * dt;
-                    double sd = __dmul_rn(fn[1], xp[0]);
-                    sd = __dadd_rn(sd, __dmul_rn(fn[2], xp[1]));
-                    sd = __dadd_rn(sd, __dmul_rn(fn[3], 0.0));
-                    sd = __dsub_rn(sd, fn[4]);
-                    sd = __dsub_rn(sd, __dmul_rn(fn[5], tt));
-#pragma unroll
-                    for (int v = 0; v < 5; v++) bs[v] = (sd < 0.0) ? fn[6 + v] : fn[11 + v];
-                }
-                const double lb = boundary_flux_vn<DIM>(bt, nvec, so, bs, P, quirk3d, F);
-                lam = (lam < lb) ? lb : lam;
-                if constexpr (AXI) {
-                    // dU_face1 *= r (BdrFaceIntegrator.cpp:109-111)
-                    const double rf = sR[ej][no];
-#pragma unroll
-                    for (int v = 0; v < NV; v++) F[v] *= rf;
-                }
-                double d[NV];
-#pragma unroll
-                for (int v = 0; v < NV; v++) d[v] = -F[v];
-                if (A.parabolic && (bt == BC_OUTFLOW || bt == BC_NOSLIP)) {
-                    double fn[NV];
-#pragma unroll
-                    for (int v = 1; v < NV; v++) fn[v] = (double)fvfp[(efo * (NV - 1) + (v - 1)) * NFP + l];
-                    if (bt == BC_NOSLIP) {
-                        double en = bs[0] * fn[1], nn2 = nvec[0] * nvec[0];
-#pragma unroll
-                        for (int d = 1; d < DIM; d++) {
-                            en = en + bs[d] * fn[1 + d];
-                            nn2 = nn2 + nvec[d] * nvec[d];
-                        }
-                        fn[NV - 1] = en + bs[3] * sqrt(nn2);
-                    }
-#pragma unroll
-                    for (int v = 1; v < NV; v++) d[v] += fn[v];
-                }
-#pragma unroll
-                for (int v = 0; v < NV; v++) sFc[ej][v][rem] = d[v];
-                continue;
-            }
-            const int gn = A.geo.fnb[efo * NFP + l];
-            if constexpr (AXI) {
-                axis_node(A.y, A.geo, K, NK, (size_t)gn, pn);
-            } else {
-#pragma unroll
-                for (int v = 0; v < NV; v++) pn[v] = A.y[v * NK + (size_t)gn];
-            }
-            const bool own = code & 1;
-            // the face's first and second states, element by element (not a
-            // pointer to one of the two arrays, which would put both in
-            // scratch memory)
-            double g1[NV], g2[NV];
-#pragma unroll
-            for (int v = 0; v < NV; v++) {
-                g1[v] = own ? so[v] : pn[v];
-                g2[v] = own ? pn[v] : so[v];
-            }
-            double fvn[NV];
-            fvn[0] = 0.0;
-            if (A.parabolic) {
-                const int nf = A.geo.fnf[efo];
-                const size_t fid = (size_t)(nf >> 1);
-                int l2;
-                if constexpr (DIM == 2) l2 = (nf & 1) ? NP - 1 - l : l;
-                else l2 = face_point_3<NP>(gn - (int)(fid / 6) * K, (int)(fid % 6) >> 1);
-#pragma unroll
-                for (int v = 1; v < NV; v++)
-                    fvn[v] = ((double)fvfp[(efo * (NV - 1) + (v - 1)) * NFP + l] +
-                              (double)fvfp[(fid * (NV - 1) + (v - 1)) * NFP + l2]) * 0.5;
-                if (A.quirks) {
-                    // ComputeViscousFlux left velocities in the momentum slots
-                    // (DGSEMIntegrator.cpp:471-481)
-                    const double r1 = 1.0 / g1[0], r2 = 1.0 / g2[0];
-#pragma unroll
-                    for (int d = 0; d < DIM; d++) { g1[1 + d] *= r1; g2[1 + d] *= r2; }
-                }
-            }
-            const NodeQ<DIM> q1 = node_quants<DIM>(g1, P);
-            const NodeQ<DIM> q2 = node_quants<DIM>(g2, P);
-            ec_flux<DIM, true>(nvec, norml2_v<DIM>(nvec), q1, q2, P, quirk3d, F);
-            if constexpr (AXI) {
-                // flux_num *= r (DGSEMIntegrator.cpp:190-205), the r of the
-                // first element's node on both sides
-                // (both values read, then chosen: a choice between the two
-                // loads compiles to one flat load through a selected address)
-                const double rl = sR[ej][no], rg = A.geo.rnode[gn];
-                const double rf = own ? rl : rg;
-#pragma unroll
-                for (int v = 0; v < NV; v++) F[v] *= rf;
-            }
-#pragma unroll
-            for (int v = 0; v < NV; v++) {
-                double d;
-                if (A.parabolic) d = own ? (-F[v] + fvn[v]) : (F[v] - fvn[v]);
-                else d = own ? -F[v] : F[v];
-                sFc[ej][v][rem] = d;
-            }
-            continue;
+        for (int v = 0; v < NV; v++) {
+            pn[v] = A.y[v * NK + (size_t)en * NP + (side ? 0 : NP - 1)];
+            so[v] = sU[ej][v][no];
         }
         if constexpr (OPEN) {
             // boundary point: -F_b for the outward normal at the interior
             // node (BdrFaceIntegrator.cpp:61-123, applied after the interior
             // faces by DGSEMNonlinearForm.cpp:776-826); its wave speed joins
             // the running maximum (DGSEMOperator.cpp:585-589)
-            const int bt = boundary_of(A.geo, eo, r, side);
+            const int bt = boundary_of(A.geo, eo, 0, side);
             if (bt != BC_PERIODIC) {
-                double F[NV];
-                const double ns = side ? nr : -nr;
-                // the side's outer state as values: a select between the
-                // table and the interior state would otherwise become one
-                // load through a selected pointer, keeping so in scratch
                 double bs[5];
 #pragma unroll
-                for (int v = 0; v < 5; v++) bs[v] = A.geo.bcs[(2 * r + side) * 5 + v];
-                const double lb = boundary_flux<DIM>(bt, r, ns, nr, so, bs, P, quirk3d, F);
+                for (int v = 0; v < 5; v++) bs[v] = A.geo.bcs[side * 5 + v];
+                const double lb = boundary_flux<1>(bt, 0, side ? nr : -nr, nr, so, bs, P, false, F);
                 lam = (lam < lb) ? lb : lam;
-                double d[NV];
 #pragma unroll
-                for (int v = 0; v < NV; v++) d[v] = -F[v];
-                if (A.parabolic && (bt == BC_OUTFLOW || bt == BC_NOSLIP)) {
-                    // + Fv.n of the interior state and gradients (this
-                    // element's trace from k_visc); inflow and specified
-                    // states have zero gradients, so no viscous flux
-                    // (BdrFaceIntegrator.cpp:141-175); the no-slip wall's energy
-                    // term is V.(Fv.n)_mom + qn |n|
-                    double fn[NV];
-#pragma unroll
-                    for (int v = 1; v < NV; v++) fn[v] = pfo[v] * ns;
-                    if (bt == BC_NOSLIP) {
-                        double en = bs[0] * fn[1];
-#pragma unroll
-                        for (int dd = 1; dd < DIM; dd++) en = en + bs[dd] * fn[1 + dd];
-                        fn[NV - 1] = en + bs[3] * sqrt(ns * ns);
-                    }
-#pragma unroll
-                    for (int v = 1; v < NV; v++) d[v] += fn[v];
-                }
-#pragma unroll
-                for (int v = 0; v < NV; v++) sFc[ej][v][rem] = d[v];
+                for (int v = 0; v < NV; v++) sF[ej][v][side] = -F[v];
                 continue;
             }
         }
@@ -978,250 +628,96 @@ __device__ __forceinline__ void rhs_body(const KArgs &A, const int tile, const i
             s1[v] = side ? so[v] : pn[v];
             s2[v] = side ? pn[v] : so[v];
         }
-        double fvn[NV];
-        fvn[0] = 0.0;
-        if (A.parabolic) {
+        const NodeQ<1> q1 = node_quants<1>(s1, P), q2 = node_quants<1>(s2, P);
+        if (A.ec) ec_flux<1, false>(&nr, nr, q1, q2, P, false, F);
+        else ec_flux<1, true>(&nr, nr, q1, q2, P, false, F);
 #pragma unroll
-            for (int v = 1; v < NV; v++) fvn[v] = ((pfo[v] + pfn[v]) * 0.5) * nr;
-            if (A.quirks) {
-                // ComputeViscousFlux left velocities in the momentum slots of
-                // state1/state2 (DGSEMIntegrator.cpp:471-481)
-                const double r1 = 1.0 / s1[0], r2 = 1.0 / s2[0];
+        for (int v = 0; v < NV; v++) sF[ej][v][side] = side ? -F[v] : F[v];
+    }
+    block_lam_max<BLOCK>(lam, lam_old, A.lam, sRed, blockIdx.x);
+    __syncthreads();
+    double accS[NV], accV[NV], accF[NV];
 #pragma unroll
-                for (int d = 0; d < DIM; d++) { s1[1 + d] *= r1; s2[1 + d] *= r2; }
-            }
-        }
-        const NodeQ<DIM> q1 = node_quants<DIM>(s1, P);
-        const NodeQ<DIM> q2 = node_quants<DIM>(s2, P);
+    for (int v = 0; v < NV; v++) {
+        accS[v] = accV[v] = accF[v] = 0.0;
+        if (act && n == 0) accS[v] += A.geo.aface * sF[el][v][0];
+        if (act && n == NP - 1) accS[v] += A.geo.aface * sF[el][v][1];
+    }
+    __syncthreads();
+
+    // ---- symmetric volume pairs (a < b) and subcell FV interfaces ----
+    for (int j = t; j < EPB * JOBS; j += BLOCK) {
+        // pairs of all elements first, then the interfaces
+        const bool pair = j < EPB * NPAIR;
+        const int jj = pair ? j : j - EPB * NPAIR;
+        const int ej = pair ? jj / NPAIR : jj / cmx(NFV, 1);
+        if (ebase + ej >= NE) continue;
         double F[NV];
-        double nvec[DIM];
+        if (pair) {
+            const int p = jj - ej * NPAIR;
+            int a, b;
+            pair_ab<NP>(p, a, b);
+            NodeQ<1> qa, qb;
+            qa.rho = sU[ej][0][a]; qb.rho = sU[ej][0][b];
+            qa.v[0] = sQ[ej][0][a]; qb.v[0] = sQ[ej][0][b];
+            qa.beta = sQ[ej][1][a]; qb.beta = sQ[ej][1][b];
+            ec_flux<1, false>(&nr, nr, qa, qb, P, false, F);
 #pragma unroll
-        for (int d = 0; d < DIM; d++) nvec[d] = (d == r) ? nr : 0.0;
-        if (A.ec) ec_flux<DIM, false>(nvec, nr, q1, q2, P, false, F);
-        else ec_flux<DIM, true>(nvec, nr, q1, q2, P, quirk3d, F);
+            for (int v = 0; v < NV; v++) sF[ej][v][p] = F[v];
+        } else if constexpr (BLEND) {
+            const int i = jj - ej * NFV;
+            if (!(sAl[ej] > 0.0)) {
+#pragma unroll
+                for (int v = 0; v < NV; v++) sF[ej][v][NPAIR + i] = 0.0;
+                continue;
+            }
+            NodeQ<1> qa, qb;
+            qa.rho = sU[ej][0][i]; qb.rho = sU[ej][0][i + 1];
+            qa.v[0] = sQ[ej][0][i]; qb.v[0] = sQ[ej][0][i + 1];
+            qa.beta = sQ[ej][1][i]; qb.beta = sQ[ej][1][i + 1];
+            qa.ibeta = sQ[ej][NQ - 2][i]; qb.ibeta = sQ[ej][NQ - 2][i + 1];
+            qa.lam = sQ[ej][NQ - 1][i]; qb.lam = sQ[ej][NQ - 1][i + 1];
+            ec_flux<1, true>(&sSub[i], sSub[i], qa, qb, P, false, F);
+#pragma unroll
+            for (int v = 0; v < NV; v++) sF[ej][v][NPAIR + i] = F[v];
+        }
+    }
+    __syncthreads();
+    if (!act) return;   // no barrier follows
+#pragma unroll
+    for (int m = 0; m < NP; m++) {
+        if (m == n) continue;
+        const double dm = sDh2[n * NP + m];
+        const int p = m < n ? pair_index<NP>(m, n) : pair_index<NP>(n, m);
+#pragma unroll
+        for (int v = 0; v < NV; v++) accV[v] += dm * sF[el][v][p];
+    }
+    if (BLEND && alpha_e > 0.0) {
+        const double fvs = sFvs[n];
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            double d;
-            if (A.parabolic) d = side ? (-F[v] + fvn[v]) : (F[v] - fvn[v]);
-            else d = side ? -F[v] : F[v];
-            sFc[ej][v][rem] = d;
-        }
-    }
-
-    // the block's wave speed: every contribution (nodes, boundary points) is
-    // in by now, and reducing it here keeps it out of the registers the pair
-    // phase needs
-    block_lam_max<BLOCK>(lam, lam_old, A.lam, sRed, slot);
-
-    double accV[NV], accS[NV], accF[NV];
-#pragma unroll
-    for (int v = 0; v < NV; v++) { accV[v] = 0.0; accS[v] = 0.0; accF[v] = 0.0; }
-    double u0v[NV], vis[NV];
-
-    // this node's surface terms, faces in direction order, low side first
-    __syncthreads();
-    const double aface = GEN ? 1.0 / (A.tab.w[0] * jn) : A.geo.aface;
-    if (act) {
-#pragma unroll
-        for (int r = 0; r < DIM; r++) {
-            const int l = line_of<DIM, NP>(r, ii[0], ii[1], ii[2]);
-            if (ii[r] == 0)
-#pragma unroll
-                for (int v = 0; v < NV; v++) accS[v] += aface * sFc[el][v][(2 * r) * NFP + l];
-            if (ii[r] == NP - 1)
-#pragma unroll
-                for (int v = 0; v < NV; v++) accS[v] += aface * sFc[el][v][(2 * r + 1) * NFP + l];
-        }
-    }
-    __syncthreads();
-
-    for (int r = 0; r < DIM; r++) {
-        const double nr = A.geo.nrm[r];
-        double nvr[DIM];   // the box's metric vector of direction r
-#pragma unroll
-        for (int d = 0; d < DIM; d++) nvr[d] = (d == r) ? nr : 0.0;
-        if (PREFETCH && r == DIM - 1 && act) {
-            // inputs of the final assembly, in flight during the last direction
-#pragma unroll
-            for (int v = 0; v < NV; v++) {
-                u0v[v] = (A.mode == 2) ? A.u0[v * NK + (size_t)e * K + n] : 0.0;
-                vis[v] = (A.parabolic && v > 0)
-                             ? (double)static_cast<const VT *>(A.visc)[(v - 1) * NK + (size_t)e * K + n] : 0.0;
-            }
-        }
-        for (int l0 = 0; l0 < NFP; l0 += LC) {
-            const int npj = EPB * LC * NPAIR, nvj = EPB * LC * NFV;
-            for (int j = t; j < npj + nvj; j += BLOCK) {
-                if (j < npj) {
-                    // ---- symmetric volume pair (a < b) on line l ----
-                    const int ej = j / (LC * NPAIR);
-                    const int rem = j - ej * (LC * NPAIR);
-                    const int lc = rem / NPAIR, p = rem - lc * NPAIR;
-                    if (ebase + ej >= NE) continue;
-                    int a, b;
-                    pair_ab<NP>(p, a, b);
-                    const int na = line_node<DIM, NP>(r, l0 + lc, a);
-                    const int nb = line_node<DIM, NP>(r, l0 + lc, b);
-                    NodeQ<DIM> qa, qb;
-                    qa.rho = sU[ej][0][na]; qb.rho = sU[ej][0][nb];
-#pragma unroll
-                    for (int d = 0; d < DIM; d++) { qa.v[d] = sQ[ej][d][na]; qb.v[d] = sQ[ej][d][nb]; }
-                    qa.beta = sQ[ej][DIM][na]; qb.beta = sQ[ej][DIM][nb];
-                    double F[NV];
-                    if constexpr (GEN) {
-                        // ComputeVolumeFlux with the mean of the two adjugate rows
-                        double mm[DIM];
-#pragma unroll
-                        for (int d = 0; d < DIM; d++) mm[d] = (sM[ej][DIM * r + d][na] + sM[ej][DIM * r + d][nb]) * 0.5;
-                        ec_flux<DIM, false>(mm, 0.0, qa, qb, P, false, F);
-                        if constexpr (AXI) {
-                            // f *= r_hat, r at the pair's midpoint (DGSEMIntegrator.cpp:272-292)
-                            const double rh = (sR[ej][na] + sR[ej][nb]) * 0.5;
-#pragma unroll
-                            for (int v = 0; v < NV; v++) F[v] *= rh;
-                        }
-                    } else {
-                        ec_flux<DIM, false>(nvr, nr, qa, qb, P, false, F);
-                    }
-#pragma unroll
-                    for (int v = 0; v < NV; v++) sF[ej][v][lc * NPAIR + p] = F[v];
-                    if (QNS3 && r == 1 && b == NP - 1)
-#pragma unroll
-                        for (int v = 0; v < NV; v++) sG[ej][v][na] = F[v];
-                } else if constexpr (BLEND) {
-                    // ---- subcell FV interface i+1/2 on line l ----
-                    const int jv = j - npj;
-                    const int ej = jv / (LC * NFV);
-                    const int rem = jv - ej * (LC * NFV);
-                    const int lc = rem / NFV, i = rem - lc * NFV;
-                    if (ebase + ej >= NE) continue;
-                    const int slot = LC * NPAIR + lc * NFV + i;
-                    if (!(sAl[ej] > 0.0)) {
-#pragma unroll
-                        for (int v = 0; v < NV; v++) sF[ej][v][slot] = 0.0;
-                        continue;
-                    }
-                    const int na = line_node<DIM, NP>(r, l0 + lc, i);
-                    const int nb = line_node<DIM, NP>(r, l0 + lc, i + 1);
-                    NodeQ<DIM> qa, qb;
-                    qa.rho = sU[ej][0][na]; qb.rho = sU[ej][0][nb];
-#pragma unroll
-                    for (int d = 0; d < DIM; d++) { qa.v[d] = sQ[ej][d][na]; qb.v[d] = sQ[ej][d][nb]; }
-                    qa.beta = sQ[ej][DIM][na]; qb.beta = sQ[ej][DIM][nb];
-                    qa.ibeta = sQ[ej][NQ - 2][na]; qb.ibeta = sQ[ej][NQ - 2][nb];
-                    qa.lam = sQ[ej][NQ - 1][na]; qb.lam = sQ[ej][NQ - 1][nb];
-                    double F[NV];
-                    if constexpr (GEN) {
-                        const double *sn = A.geo.subn + (((((size_t)(ebase + ej) * DIM + r) * NFP + l0 + lc) * (NP - 1) + i) * DIM);
-                        double nv2[DIM];
-#pragma unroll
-                        for (int d = 0; d < DIM; d++) nv2[d] = sn[d];
-                        ec_flux<DIM, true>(nv2, norml2_v<DIM>(nv2), qa, qb, P, quirk3d, F);
-                        if constexpr (AXI) {
-                            // flux_num *= mid_r (DGSEMIntegrator.cpp:1030-1032, 1110-1112)
-                            const double rh = (sR[ej][na] + sR[ej][nb]) * 0.5;
-#pragma unroll
-                            for (int v = 0; v < NV; v++) F[v] *= rh;
-                        }
-                    } else {
-                        double nv2[DIM];
-#pragma unroll
-                        for (int d = 0; d < DIM; d++) nv2[d] = (d == r) ? sSub[r][i] : 0.0;
-                        ec_flux<DIM, true>(nv2, sSub[r][i], qa, qb, P, quirk3d, F);
-                    }
-#pragma unroll
-                    for (int v = 0; v < NV; v++) sF[ej][v][slot] = F[v];
-                }
-            }
-            __syncthreads();
-            if (act) {
-                const int l = line_of<DIM, NP>(r, ii[0], ii[1], ii[2]);
-                if (l >= l0 && l < l0 + LC) {
-                    const int lc = l - l0;
-                    const int a = ii[r];
-#pragma unroll
-                    for (int m = 0; m < NP; m++) {
-                        if (m == a) continue;
-                        const double dm = sDh2[a * NP + m];
-                        if (QNS3 && r == 2 && m < a) {
-                            // H_inviscid(id2).SetCol(k, g) (DGSEMIntegrator.cpp:702)
-                            const int nm = line_node<DIM, NP>(r, l, m);
-#pragma unroll
-                            for (int v = 0; v < NV; v++) accV[v] += dm * sG[el][v][nm];
-                        } else {
-                            const int p = m < a ? pair_index<NP>(m, a) : pair_index<NP>(a, m);
-#pragma unroll
-                            for (int v = 0; v < NV; v++) accV[v] += dm * sF[el][v][lc * NPAIR + p];
-                        }
-                    }
-                    if (BLEND && alpha_e > 0.0) {
-                        const int base = LC * NPAIR + lc * NFV;
-                        // 1/(J_i w_i) (DGSEMIntegrator.cpp:1046) with this node's J
-                        const double fvs = GEN ? 1.0 / (jn * A.tab.w[a]) : sFvs[a];
-#pragma unroll
-                        for (int v = 0; v < NV; v++) {
-                            double val;
-                            if (a == 0) val = (0.0 - sF[el][v][base + 0]) * fvs;
-                            else if (a == NP - 1) val = sF[el][v][base + NP - 2] * fvs;
-                            else val = (sF[el][v][base + a - 1] - sF[el][v][base + a]) * fvs;
-                            accF[v] = (r == 0) ? val : accF[v] + val;
-                        }
-                    }
-                }
-            }
-            __syncthreads();
+            const double lo = n > 0 ? sF[el][v][NPAIR + n - 1] : 0.0;
+            const double hi = n < NP - 1 ? sF[el][v][NPAIR + n] : 0.0;
+            accF[v] = (lo - hi) * fvs;
         }
     }
 
     // ---- assemble, stage update, store ----
-    if (!PREFETCH && act) {
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-            u0v[v] = (A.mode == 2) ? A.u0[v * NK + (size_t)e * K + n] : 0.0;
-            vis[v] = (A.parabolic && v > 0)
-                         ? (double)static_cast<const VT *>(A.visc)[(v - 1) * NK + (size_t)e * K + n] : 0.0;
-        }
-    }
-    if (act) {
-        double src = 0.0;
-        if constexpr (AXI) {
-            // PressureFromConservative (DGSEMIntegrator.cpp:1306-1315) of this node
-            const double ke = 0.5 * ((sU[el][1][n] * sU[el][1][n] + sU[el][2][n] * sU[el][2][n]) / sU[el][0][n]);
-            src = P.gm1 * (sU[el][3][n] - ke);
-        }
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            double vol = -accV[v];
-            if (BLEND) vol *= (1.0 - alpha_e);
-            if (A.parabolic && v > 0) vol = vol + vis[v];
-            vol *= GEN ? 1.0 / jn : A.geo.invJ;
-            double tot = (BLEND && alpha_e > 0.0) ? accF[v] * alpha_e + vol : vol;
-            if (AXI && v == 2) tot += src;   // DGSEMIntegrator.cpp:411-426
-            tot += accS[v];
-            // ZeroAxisRadialMom (DGSEMOperator.cpp:521-533)
-            if (AXI && v == 2 && axown >= 0 && (axown & 1)) tot = 0.0;
-            const size_t gi = v * NK + (size_t)e * K + n;
-            const double yv = AXI ? yw[v] : sU[el][v][n];
-            double o;
-            if (A.mode == 0) o = tot;
-            else if (A.mode == 1) o = yv + dt * tot;
-            else o = A.c0 * u0v[v] + A.c1 * (yv + dt * tot);
-            A.out[gi] = o;
-        }
+    for (int v = 0; v < NV; v++) {
+        double vol = -accV[v];
+        if (BLEND) vol *= (1.0 - alpha_e);
+        vol *= A.geo.invJ;
+        const double tot = ((BLEND && alpha_e > 0.0) ? accF[v] * alpha_e + vol : vol) + accS[v];
+        const size_t gi = v * NK + (size_t)e * NP + n;
+        const double yv = sU[el][v][n];
+        double o;
+        if (A.mode == 0) o = tot;
+        else if (A.mode == 1) o = yv + dt * tot;
+        else o = A.c0 * A.u0[gi] + A.c1 * (yv + dt * tot);
+        A.out[gi] = o;
     }
 }
-
-// OPEN: the box has non-periodic sides (Euler, natural shape); the periodic
-// kernels carry no boundary code.  GEN: a quadrilateral or hexahedral mesh.
-template <int DIM, int NP, bool BLEND, bool QNS3, typename VT, int FB, bool OPEN = false, bool GEN = false,
-          bool AXI = false>
-__global__ void __launch_bounds__((RCfg<DIM, NP, BLEND, FB>::BLOCK))
-__attribute__((amdgpu_waves_per_eu(RCfg<DIM, NP, BLEND, FB>::WAVES))) k_rhs(const KArgs A)
-{
-    __shared__ RhsSmem<DIM, NP, BLEND, QNS3, FB, GEN, AXI> S;
-    rhs_body<DIM, NP, BLEND, QNS3, VT, FB, OPEN, GEN, AXI>(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.x, S);
-}
-
 
 // ---------------------------------------------------------------------------
 // k_visc: entropy variables, BR1 lifting, gradient conversion, viscous fluxes

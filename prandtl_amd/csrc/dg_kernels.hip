@@ -44,9 +44,9 @@ struct EnsTile {
     int v;   // variant: 2*(NP-3) + blend
 };
 
-constexpr int ENS_BLOCK = 256;
+constexpr int ENS_BLOCK = 64;   // the 2-D line tiles' workgroup, one wave
 
-template <int NP, bool BLEND> constexpr size_t ens_smem() { return sizeof(RhsSmem<2, NP, BLEND, false, ENS_BLOCK>); }
+template <int NP, bool BLEND> constexpr size_t ens_smem() { return sizeof(LineSmem<2, NP, BLEND, 0, false, false>); }
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
 constexpr size_t ENS_SMEM = cmax(cmax(cmax(ens_smem<3, false>(), ens_smem<3, true>()), cmax(ens_smem<4, false>(), ens_smem<4, true>())),
                                  cmax(cmax(ens_smem<5, false>(), ens_smem<5, true>()), cmax(ens_smem<6, false>(), ens_smem<6, true>())));
@@ -54,8 +54,8 @@ constexpr size_t ENS_SMEM = cmax(cmax(cmax(ens_smem<3, false>(), ens_smem<3, tru
 template <int NP, bool BLEND>
 __device__ __forceinline__ void ens_tile(const KArgs &A, int g, double *smem, int tid = -1)
 {
-    rhs_body<2, NP, BLEND, false, double, ENS_BLOCK>(A, g, g, *reinterpret_cast<RhsSmem<2, NP, BLEND, false, ENS_BLOCK> *>(smem),
-                                                     tid);
+    static_assert(LnCfg<2, NP>::BLOCK == ENS_BLOCK, "one workgroup size for every tile");
+    line_body<2, NP, BLEND, false, double, 0>(A, g, g, *reinterpret_cast<LineSmem<2, NP, BLEND, 0, false, false> *>(smem), tid);
 }
 
 // grid = number of tiles; every field of a tile is uniform over the workgroup
@@ -96,7 +96,7 @@ k_ens(const KArgs *__restrict__ cases, const EnsTile *__restrict__ tiles)
 //  - the tile index read back from LDS goes through readfirstlane, so the
 //    tile's fields, the variant branch and the case's arguments are scalar
 //    as in k_ens.
-__global__ void __launch_bounds__(ENS_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(ENS_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
 k_ens_q(const KArgs *__restrict__ cases, const EnsTile *__restrict__ tiles, int ntiles, int *counter)
 {
     __shared__ __align__(16) double smem[(ENS_SMEM + 7) / 8];
@@ -706,7 +706,6 @@ int create_impl(const prandtl_mesh_desc *mesh, const prandtl_quad_mesh *qm, cons
         }
         // the kernels recompute the per-node metrics from the corners
         qg.met.clear();
-        qg.jac.clear();
         c->gen = true;
         c->hmin = qg.hmin;
     }
@@ -818,7 +817,7 @@ int create_impl(const prandtl_mesh_desc *mesh, const prandtl_quad_mesh *qm, cons
         c->geo.fface = reinterpret_cast<const int *>(b + off[5]);
         c->geo.fnb = reinterpret_cast<const int *>(b + off[6]);
         c->geo.fnf = reinterpret_cast<const int *>(b + off[7]);
-        if (hm) c->geo.corner = reinterpret_cast<const double *>(b + off[12]);
+        c->geo.corner = reinterpret_cast<const double *>(b + off[12]);
         if (qm) c->geo.fxy = reinterpret_cast<const double *>(b + off[13]);
         c->nattr = qm ? qm->nattr : hm->nattr;
         if (c->axi) {
@@ -1645,14 +1644,14 @@ namespace {
 int ens_epb(int NP, int blend)
 {
     switch (NP * 2 + blend) {
-    case 6: return RCfg<2, 3, false, ENS_BLOCK>::EPB;
-    case 7: return RCfg<2, 3, true, ENS_BLOCK>::EPB;
-    case 8: return RCfg<2, 4, false, ENS_BLOCK>::EPB;
-    case 9: return RCfg<2, 4, true, ENS_BLOCK>::EPB;
-    case 10: return RCfg<2, 5, false, ENS_BLOCK>::EPB;
-    case 11: return RCfg<2, 5, true, ENS_BLOCK>::EPB;
-    case 12: return RCfg<2, 6, false, ENS_BLOCK>::EPB;
-    case 13: return RCfg<2, 6, true, ENS_BLOCK>::EPB;
+    case 6: return LnCfg<2, 3>::EPB;
+    case 7: return LnCfg<2, 3>::EPB;
+    case 8: return LnCfg<2, 4>::EPB;
+    case 9: return LnCfg<2, 4>::EPB;
+    case 10: return LnCfg<2, 5>::EPB;
+    case 11: return LnCfg<2, 5>::EPB;
+    case 12: return LnCfg<2, 6>::EPB;
+    case 13: return LnCfg<2, 6>::EPB;
     default: return 0;
     }
 }
@@ -1707,7 +1706,7 @@ void ens_stage(prandtl_ensemble *E, int k, int mode, hipStream_t s)
     if (mode == 0)
         hipLaunchKernelGGL(k_ens, dim3(E->ntiles), dim3(ENS_BLOCK), 0, s, E->d_args[k], E->d_tiles);
     else
-        hipLaunchKernelGGL(k_ens_q, dim3(mode * E->ncu), dim3(ENS_BLOCK), 0, s, E->d_args[k], E->d_tiles, E->ntiles,
+        hipLaunchKernelGGL(k_ens_q, dim3(4 * mode * E->ncu), dim3(ENS_BLOCK), 0, s, E->d_args[k], E->d_tiles, E->ntiles,
                            E->d_counters + k);
 }
 

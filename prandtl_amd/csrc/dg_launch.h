@@ -5,8 +5,7 @@
 #include <string>
 #include <vector>
 #include "dg_device.h"
-#include "dg_line.h"
-#include "dg_line_high.h"
+#include "dg_lines.h"
 #include "dg_visc_mx.h"
 
 using namespace prandtl;
@@ -187,145 +186,92 @@ template <int DIM, int NP> int launch_visc(prandtl_ctx *c, const double *y, doub
     else return launch_visc_nd<DIM, NP>(c, y, grad, s);
 }
 
-template <int DIM, int NP, bool BLEND, int FB>
-void launch_rhs_fb(prandtl_ctx *c, const KArgs &a, hipStream_t s)
-{
-    using Cf = RCfg<DIM, NP, BLEND, FB>;
-    const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-    if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED)
-        hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, float, FB>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-    else hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, double, FB>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-}
-
-// The line kernel serves periodic Cartesian boxes of the orders line_built
-// lists.
+// The orders whose periodic 3-D boxes have a choice of algorithm (N = 2..4).
+constexpr bool line_built(int DIM, int NP) { return DIM == 3 && NP >= 3 && NP <= 5; }
 inline bool line_ok(const prandtl_ctx *c)
 {
     return line_built(c->dim, c->Np) && !c->gen && !c->axi && c->geo.bcmask == 0;
 }
 
-// The default algorithm where the line kernel exists: it is the faster one
-// at N = 2 and 3, and with blending at N = 4; unblended N = 4 runs the tile
-// kernel faster (12^3 boxes on MI355X: Euler 35.6 against 42.0 us per RHS,
-// Navier-Stokes 54.9 against 62.3).
+// The default there.  Both values run k_rhs_l; LINE adds k_visc_mx in the
+// mixed form at N = 3, TILE the forced launch shapes.
 inline bool line_default(const prandtl_ctx *c)
 {
     return line_ok(c) && (c->Np <= 4 || c->prm.blending);
 }
 
-template <int DIM, int NP, bool BLEND>
-int launch_rhs_low(prandtl_ctx *c, const KArgs &a, hipStream_t s)
+// One instance of k_rhs_l: the faithful NS-3D form, the mixed form or plain FP64.
+template <int DIM, int NP, bool BLEND, int FB, bool OPEN, bool GEN>
+int launch_lines(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
-    const bool qns3 = DIM == 3 && c->prm.parabolic && c->prm.quirks;
-    if constexpr (line_built(DIM, NP)) {
-        if (c->rhs_algo == PRANDTL_ALGO_LINE && line_ok(c)) {
-            using Lc = LCfg<DIM, NP>;
-            const int nb = (c->NE + Lc::EPB - 1) / Lc::EPB;
-            if (qns3)
-                hipLaunchKernelGGL((k_rhs_ln<DIM, NP, BLEND, true, double>), dim3(nb), dim3(Lc::BLOCK), 0, s, a);
-            else if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED)
-                hipLaunchKernelGGL((k_rhs_ln<DIM, NP, BLEND, false, float>), dim3(nb), dim3(Lc::BLOCK), 0, s, a);
-            else hipLaunchKernelGGL((k_rhs_ln<DIM, NP, BLEND, false, double>), dim3(nb), dim3(Lc::BLOCK), 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_rhs_ln launch");
+    using Lc = LnCfg<DIM, NP, FB>;
+    const dim3 nb((c->NE + Lc::EPB - 1) / Lc::EPB), bl(Lc::BLOCK);
+    if constexpr (DIM == 2 && GEN) {
+        if (c->axi) {
+            // the axisymmetric RHS (Euler), recovering U from r U as it loads
+            hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, double, FB, OPEN, GEN, true>), nb, bl, 0, s, a);
+            return hip_check(c, hipGetLastError(), "k_rhs_l launch");
         }
     }
-    if constexpr (gen_built(DIM, NP)) {
-        if (c->gen) {
-            // quadrilateral or hexahedral mesh, natural shape
-            using Cf = RCfg<DIM, NP, BLEND>;
-            const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-            if constexpr (DIM == 2) {
-                if (c->axi) {
-                    // the axisymmetric RHS (Euler), recovering U from r U as it loads
-                    hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, double, 0, false, true, true>), dim3(nb),
-                                       dim3(Cf::BLOCK), 0, s, a);
-                    return hip_check(c, hipGetLastError(), "k_rhs launch");
-                }
-            } else {
-                if (qns3) {
-                    // the faithful NS-3D form on a hexahedral mesh
-                    hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, true, double, 0, false, true>), dim3(nb),
-                                       dim3(Cf::BLOCK), 0, s, a);
-                    return hip_check(c, hipGetLastError(), "k_rhs launch");
-                }
-            }
-            if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED)
-                hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, float, 0, false, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-            else hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, double, 0, false, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_rhs launch");
+    if constexpr (DIM == 3) {
+        if (c->prm.parabolic && c->prm.quirks) {
+            hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, true, double, FB, OPEN, GEN>), nb, bl, 0, s, a);
+            return hip_check(c, hipGetLastError(), "k_rhs_l launch");
         }
     }
-    if (c->geo.bcmask) {
-        // boundary sides, natural shape
-        using Cf = RCfg<DIM, NP, BLEND>;
-        const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-        if constexpr (DIM == 3) {
-            if (qns3) {
-                // the faithful NS-3D form with boundary sides
-                hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, true, double, 0, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-                return hip_check(c, hipGetLastError(), "k_rhs launch");
-            }
+    if constexpr (DIM > 1) {
+        if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED) {
+            hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, float, FB, OPEN, GEN>), nb, bl, 0, s, a);
+            return hip_check(c, hipGetLastError(), "k_rhs_l launch");
         }
-        if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED)
-            hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, float, 0, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-        else hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, false, double, 0, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-        return hip_check(c, hipGetLastError(), "k_rhs launch");
     }
-    if (qns3) {
-        // the faithful NS-3D form runs in the natural shape only
-        using Cf = RCfg<DIM, NP, BLEND>;
-        const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-        hipLaunchKernelGGL((k_rhs<DIM, NP, BLEND, DIM == 3, double, 0>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-        return hip_check(c, hipGetLastError(), "k_rhs launch");
-    }
-    switch (c->rhs_shape) {
-    case 1:
-        if constexpr (rhs_shape_ok(DIM, NP, BLEND, 1)) launch_rhs_fb<DIM, NP, BLEND, 64>(c, a, s);
-        break;
-    case 2:
-        if constexpr (rhs_shape_ok(DIM, NP, BLEND, 2)) launch_rhs_fb<DIM, NP, BLEND, 128>(c, a, s);
-        break;
-    case 3:
-        if constexpr (rhs_shape_ok(DIM, NP, BLEND, 3)) launch_rhs_fb<DIM, NP, BLEND, 256>(c, a, s);
-        break;
-    default:
-        launch_rhs_fb<DIM, NP, BLEND, 0>(c, a, s);
-        break;
-    }
-    return hip_check(c, hipGetLastError(), "k_rhs launch");
+    hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, double, FB, OPEN, GEN>), nb, bl, 0, s, a);
+    return hip_check(c, hipGetLastError(), "k_rhs_l launch");
 }
 
-template <int DIM, int NP, bool BLEND, int FB, bool OPEN>
-void launch_rhs_high(prandtl_ctx *c, const KArgs &a, hipStream_t s)
+// A smaller workgroup for meshes too small for the natural one: with fewer
+// natural workgroups than CUs (256), one or two elements per workgroup spread
+// over more of them.  Euler right-hand sides, natural against this: 3-D N = 3
+// 512 elements 9.3 -> 8.0 us (2,197 elements 15.7 against 14.0, 4,096 18.6
+// against 18.7), N = 4 252 elements 10.8 -> 8.9, N = 2 125 elements 10.7 -> 8.5.
+constexpr int lines_small_fb(int DIM, int NP) { return DIM != 3 || NP > 6 ? 0 : NP <= 4 ? 64 : 128; }
+
+template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN>
+int launch_lines_sized(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
-    using Hc = HCfg<DIM, NP, FB>;
-    const int nb = (c->NE + Hc::EPB - 1) / Hc::EPB;
-    if (c->prm.parabolic && c->prm.quirks)
-        hipLaunchKernelGGL((k_rhs_lh<DIM, NP, BLEND, true, double, FB, OPEN>), dim3(nb), dim3(Hc::BLOCK), 0, s, a);
-    else if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED)
-        hipLaunchKernelGGL((k_rhs_lh<DIM, NP, BLEND, false, float, FB, OPEN>), dim3(nb), dim3(Hc::BLOCK), 0, s, a);
-    else hipLaunchKernelGGL((k_rhs_lh<DIM, NP, BLEND, false, double, FB, OPEN>), dim3(nb), dim3(Hc::BLOCK), 0, s, a);
+    constexpr int SM = lines_small_fb(DIM, NP);
+    if constexpr (SM > 0) {
+        if (c->NE < 256 * LnCfg<DIM, NP>::EPB) return launch_lines<DIM, NP, BLEND, SM, OPEN, GEN>(c, a, s);
+    }
+    return launch_lines<DIM, NP, BLEND, 0, OPEN, GEN>(c, a, s);
 }
 
 template <int DIM, int NP, bool BLEND>
 int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
     ProfScope ps(c, s, 0);
-    if constexpr (high_built(DIM, NP)) {
-        if (c->geo.bcmask) launch_rhs_high<DIM, NP, BLEND, 0, true>(c, a, s);
-        else {
-            bool done = false;
-            if constexpr (rhs_shape_ok(DIM, NP, BLEND, 3)) {
-                if (c->rhs_shape == 3) {
-                    launch_rhs_high<DIM, NP, BLEND, 256, false>(c, a, s);
-                    done = true;
-                }
-            }
-            if (!done) launch_rhs_high<DIM, NP, BLEND, 0, false>(c, a, s);
+    if constexpr (DIM == 1) {
+        using Cf = R1Cfg<NP, BLEND>;
+        const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
+        if (c->geo.bcmask) hipLaunchKernelGGL((k_rhs<NP, BLEND, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+        else hipLaunchKernelGGL((k_rhs<NP, BLEND, false>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+        return hip_check(c, hipGetLastError(), "k_rhs launch");
+    } else {
+        if constexpr (gen_built(DIM, NP)) {
+            if (c->gen) return launch_lines_sized<DIM, NP, BLEND, false, true>(c, a, s);
         }
-        return hip_check(c, hipGetLastError(), "k_rhs_lh launch");
-    } else return launch_rhs_low<DIM, NP, BLEND>(c, a, s);
+        if (c->geo.bcmask) return launch_lines_sized<DIM, NP, BLEND, true, false>(c, a, s);
+        // forced shapes (a 2-D tile of 64 threads is the natural one)
+        if constexpr (DIM == 3 && rhs_shape_ok(DIM, NP, BLEND, 1))
+            if (c->rhs_shape == 1) return launch_lines<DIM, NP, BLEND, 64, false, false>(c, a, s);
+        if constexpr (rhs_shape_ok(DIM, NP, BLEND, 2))
+            if (c->rhs_shape == 2) return launch_lines<DIM, NP, BLEND, 128, false, false>(c, a, s);
+        if constexpr (rhs_shape_ok(DIM, NP, BLEND, 3))
+            if (c->rhs_shape == 3) return launch_lines<DIM, NP, BLEND, 256, false, false>(c, a, s);
+        return launch_lines_sized<DIM, NP, BLEND, false, false>(c, a, s);
+    }
 }
+
 inline KArgs make_kargs(const prandtl_ctx *c, const double *y, const double *u0, double *out, int mode,
                  double dt, double c0, double c1, const double *dtp)
 {

@@ -94,16 +94,19 @@ __device__ __forceinline__ NodeQ<DIM> node_quants(const double *s, const Phys &P
 //     series of 1/T to u^3 (the next terms are below 1e-17);
 //   u < 1/9 (y/x up to 2): T by a degree-10 polynomial, the Chebyshev
 //     interpolant of atanh(sqrt u)/sqrt u on [0, 1/9], relative error 2.4e-18;
-//   else (shocks, and every non-finite or negative value): (y-x)/log(y/x).
+//   else (shocks, and every non-finite or negative value): (y-x)/log(y/x)
+//     with log(y/x) = k log 2 + log(y/(2^k x)), k the difference of the binary
+//     exponents, which brings the second logarithm into T's range: 45
+//     instructions against 130 of the library's logarithm and quotient.
 // Largest error against an extended-precision log mean: 2.7e-16, 3.8e-16 and
-// 4.0e-16 in the three ranges; the quotient (y-x)/log(y/x) above 2%, which the
-// second range replaces, loses up to 5.3e-15 where y/x is rounded.  Next to
-// a mean by the quotient or by one rational of s and d (four divisions or
-// two reciprocals and a logarithm per pair) the fluxes of all kernels became
-// faster by: 2-D N = 4 with blending, 64^2 boxes, 38.2 -> 28.2 us per RK3
-// step's worth of right-hand sides and 2-D N = 3, 384^2, 172 -> 147 us per
-// right-hand side (shear layers, whose logarithms go); 3-D N = 3
-// Navier-Stokes, 45 x 43 x 41, 495 -> 462 us.
+// 4.3e-16 in the three ranges; the quotient (y-x)/log(y/x) of the reference
+// loses up to 5.3e-15 below a ratio of 2, where y/x is rounded.
+// Next to a mean by the quotient or by one rational of s and d (four
+// divisions or two reciprocals and a logarithm per pair) the fluxes of all
+// kernels became faster by: 2-D N = 4 with blending, 64^2 boxes, 38.2 ->
+// 28.2 us per RK3 step and 2-D N = 3, 384^2, 172 -> 147 us per right-hand
+// side (shear layers, whose logarithms go); 3-D N = 3 Navier-Stokes,
+// 45 x 43 x 41, 495 -> 462 us.
 __device__ __forceinline__ double atanh_ratio(double u)
 {
     double p = 0.08522081781390699;
@@ -119,9 +122,30 @@ __device__ __forceinline__ double atanh_ratio(double u)
     return fma(p, u, 1.0);
 }
 
-// RANGE: LM_ANY chooses per pair; LM_SHORT and LM_MID are the first two alone,
-// for callers that have bounded the ratio of a whole line's values.
-enum { LM_SHORT = 0, LM_MID = 1, LM_ANY = 2 };
+// T or log(y/x) of one mean in the third range's form: k = 0 (a ratio inside
+// (1/2, 2)) gives T(u) as the second range does; otherwise log(y/x), NaN for
+// values of different sign, as the logarithm of their quotient is.  log 2 in
+// two parts, the first with trailing zeros, so that k times it is exact.
+__device__ __forceinline__ bool log_parts(double x, double y, double &TL)
+{
+    const bool in = (y < x + x) & (x < y + y);
+    const int k = in ? 0 : __builtin_amdgcn_frexp_exp(y) - __builtin_amdgcn_frexp_exp(x);
+    const double xk = ldexp(x, k);
+    const double f = (y - xk) * rcp_nr(xk + y);
+    const double T = atanh_ratio(f * f);
+    const double kd = (double)k, f2 = f + f;
+    const double lg = fma(kd, 0.6931471803691238, f2 + fma(f2, T - 1.0, kd * 1.9082149292705877e-10));
+    TL = in ? T : (x < 0.0) != (y < 0.0) ? __builtin_nan("") : lg;
+    return in;
+}
+
+// RANGE: LM_SHORT is the first range alone, for callers that have bounded the
+// ratio of a whole line's values; LM_MID the second (and valid in the first);
+// LM_ANY every value, by the second range's formulas where they hold.  Where
+// both hold MID and ANY agree bitwise, so a wave may take ANY for all its
+// lanes as soon as one of them needs it (lm_any below) without a lane's
+// result depending on the others.
+enum { LM_SHORT = 0, LM_MID = 1, LM_ANY = 2, LM_PAIR = 3 };
 
 template <int RANGE>
 __device__ __forceinline__ void log_means(double ra, double rb, double ba, double bb, double &rho_ln,
@@ -130,22 +154,30 @@ __device__ __forceinline__ void log_means(double ra, double rb, double ba, doubl
     const double rs = ra + rb, bs = ba + bb;
     const double dr = rb - ra, db = bb - ba;
     rbs = rcp_nr(bs);
-    const double fr = dr * rcp_nr(rs), fb = db * rbs;
-    const double ur = fr * fr, ub = fb * fb;
-    if (RANGE == LM_SHORT || (RANGE == LM_ANY && ((ur < 1e-4) & (ub < 1e-4)))) {
-        // T = 1 + u/3 + u^2/5 + u^3/7, 1/T = 1 - u/3 - 4u^2/45 - 44u^3/945
-        const double tr = fma(ur, fma(ur, fma(ur, -22.0 / 945.0, -2.0 / 45.0), -1.0 / 6.0), 0.5);
-        const double tb = fma(ub, fma(ub, fma(ub, 2.0 / 7.0, 2.0 / 5.0), 2.0 / 3.0), 2.0);
-        rho_ln = rs * tr;
-        ibeta_ln = rbs * tb;
-    } else if (RANGE == LM_MID || ((ur < 1.0 / 9.0) & (ub < 1.0 / 9.0))) {
-        rho_ln = 0.5 * rs * rcp_nr(atanh_ratio(ur));
-        ibeta_ln = 2.0 * rbs * atanh_ratio(ub);
+    if constexpr (RANGE == LM_ANY) {
+        double TL;
+        bool in = log_parts(ra, rb, TL);
+        rho_ln = (in ? 0.5 * rs : dr) * rcp_nr(TL);
+        in = log_parts(ba, bb, TL);
+        ibeta_ln = (2.0 * rcp_nr(in ? bs : db)) * (in ? TL : 0.5 * TL);
     } else {
-        rho_ln = (ur < 1.0 / 9.0) ? 0.5 * rs * rcp_nr(atanh_ratio(ur)) : dr * rcp_nr(log(rb / ra));
-        ibeta_ln = (ub < 1.0 / 9.0) ? 2.0 * rbs * atanh_ratio(ub) : log(bb / ba) * rcp_nr(db);
+        const double fr = dr * rcp_nr(rs), fb = db * rbs;
+        const double ur = fr * fr, ub = fb * fb;
+        if constexpr (RANGE == LM_SHORT) {
+            // T = 1 + u/3 + u^2/5 + u^3/7, 1/T = 1 - u/3 - 4u^2/45 - 44u^3/945
+            const double tr = fma(ur, fma(ur, fma(ur, -22.0 / 945.0, -2.0 / 45.0), -1.0 / 6.0), 0.5);
+            const double tb = fma(ub, fma(ub, fma(ub, 2.0 / 7.0, 2.0 / 5.0), 2.0 / 3.0), 2.0);
+            rho_ln = rs * tr;
+            ibeta_ln = rbs * tb;
+        } else {
+            rho_ln = (0.5 * rs) * rcp_nr(atanh_ratio(ur));
+            ibeta_ln = (2.0 * rbs) * atanh_ratio(ub);
+        }
     }
 }
+
+// Whether the second range's formulas do not hold for the pair.
+__device__ __forceinline__ bool lm_outside(double x, double y) { return !((y < x + x) & (x < y + y)); }
 
 // Chandrashekar two-point flux for the normal (or mean metric) vector n.
 // DISS = false: ComputeVolumeFlux (ChandrashekarFlux.cpp:11-83).  DISS =
@@ -158,8 +190,8 @@ __device__ __forceinline__ void log_means(double ra, double rb, double ba, doubl
 //  - the momentum jump is rho_mean dv + drho v_mean, and the energy jump
 //    reuses drho h, so the conserved states are not read.
 // Symmetric in (a, b) for DISS = false, as the symmetric pairs need.
-template <int DIM, bool DISS, int RANGE = LM_ANY>
-__device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<DIM> &a, const NodeQ<DIM> &b,
+template <int DIM, bool DISS, int RANGE>
+__device__ __forceinline__ void ec_flux_r(const double *n, double nd, const NodeQ<DIM> &a, const NodeQ<DIM> &b,
                                         const Phys &P, bool quirk3d, double *F)
 {
     double rho_ln, ibeta_ln, rbs;
@@ -199,6 +231,20 @@ __device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<
         }
         F[DIM + 1] = fma(-hl, fma(drho, h, fma(0.5 * rm, e, q3)), F[DIM + 1]);
     }
+}
+
+// ec_flux_r with the range of the wave's active lanes: MID unless a lane is
+// outside it.  TRY_SHORT: lanes in the first range take it (worth the second
+// path where most waves hold such lanes only: the face points of 3-D flows).
+template <int DIM, bool DISS, bool TRY_SHORT = false>
+__device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<DIM> &a, const NodeQ<DIM> &b,
+                                        const Phys &P, bool quirk3d, double *F)
+{
+    if (TRY_SHORT && ((fabs(b.rho - a.rho) < 0.01 * (a.rho + b.rho)) & (fabs(b.beta - a.beta) < 0.01 * (a.beta + b.beta))))
+        ec_flux_r<DIM, DISS, LM_SHORT>(n, nd, a, b, P, quirk3d, F);
+    else if (__any(lm_outside(a.rho, b.rho) | lm_outside(a.beta, b.beta)))
+        ec_flux_r<DIM, DISS, LM_ANY>(n, nd, a, b, P, quirk3d, F);
+    else ec_flux_r<DIM, DISS, LM_MID>(n, nd, a, b, P, quirk3d, F);
 }
 
 // MFEM Vector::Norml2 of a 2-vector (scaled, overflow-safe), the face

@@ -498,11 +498,14 @@ bool build(const prandtl_quad_mesh *m, int order, const std::vector<double> &x,
     // per-node metrics
     const size_t NK = (size_t)NE * K;
     g.met.assign(4 * NK, 0.0);
+    g.corner.assign((size_t)NE * 8, 0.0);
     g.jac.assign(NK, 0.0);
     g.hmin = INFINITY;
     for (int e = 0; e < NE; e++) {
         double c[4][2];
         corners(e, c);
+        for (int k = 0; k < 4; k++)
+            for (int d = 0; d < 2; d++) g.corner[(size_t)e * 8 + 2 * k + d] = c[k][d];
         for (int j = 0; j < NP; j++)
             for (int i = 0; i < NP; i++) {
                 double J[2][2];

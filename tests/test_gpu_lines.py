@@ -1,4 +1,4 @@
-"""The high-order line kernel (3-D boxes of order 5..7) against the oracle:
+"""The line kernel at high order (3-D boxes of order 5..7) against the oracle:
 element counts its elements per workgroup do not divide, blended and
 unblended, Navier-Stokes in both modes and the mixed form, boundary sides;
 and the launch shapes of order 5.  The bar is the repository's parity bar
@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
-from prandtl_amd import DGSEMOperator, cases
+from prandtl_amd import DGSEMOperator, PrandtlError, cases
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +88,52 @@ def test_high_order_shapes(cuda, blend):
     op.Mult(du, b)
     torch.cuda.synchronize()
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,nelem", [(2, (12, 12, 12)), (2, (13, 12, 12)), (3, (11, 10, 9)), (3, (11, 10, 10)),
+                                     (4, (9, 9, 9)), (4, (10, 9, 9))])
+def test_line_workgroup_sizes(cuda, N, nelem):
+    """Element counts on both sides of the line below which the smaller
+    workgroup is taken (256 natural workgroups of 7, 4 and 3 elements), none
+    a multiple of every size: the natural choice and every forced shape agree
+    bitwise, and with the oracle."""
+    import torch
+    cfg = dict(dim=3, order=N, nelem=nelem, lo=(0.0,) * 3, hi=(TWO_PI, 2.0, 3.0), quirks=False, blending=True)
+    op, orc = DGSEMOperator(**cfg), O.Oracle(threads=8, **cfg)
+    X = cases.node_coords(3, N, nelem, cfg["lo"], cfg["hi"])
+    u = cases.random_smooth_state(X, 3, 37, amp=0.2, L=list(cfg["hi"]))
+    u = u * (1.0 + 0.3 * (np.arange(u.shape[1]) % 5 == 0))[None, :, None]
+    du = torch.tensor(u.reshape(-1), dtype=torch.float64, device=cuda)
+    a = torch.empty_like(du)
+    op.Mult(du, a)
+    op.set_algorithm("tile")
+    n = 0
+    for s in range(4):
+        try:
+            op.set_shape("rhs", s)
+        except PrandtlError:
+            continue
+        b = torch.empty_like(du)
+        op.Mult(du, b)
+        torch.cuda.synchronize()
+        assert torch.equal(a, b), s
+        n += 1
+    assert n >= 2
+    assert rel(a.cpu().numpy(), orc.Mult(u)) <= 1e-12
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("blend", [False, True])
+def test_line_2d_ragged(cuda, N, blend):
+    """2-D element counts that leave the last workgroup partly empty."""
+    import torch
+    cfg = dict(dim=2, order=N, nelem=(7, 5), lo=(-1.0, 0.0), hi=(1.0, 3.0), blending=blend, alpha_max=0.5)
+    op, orc = DGSEMOperator(**cfg), O.Oracle(threads=8, **cfg)
+    X = cases.node_coords(2, N, cfg["nelem"], cfg["lo"], cfg["hi"])
+    u = cases.random_smooth_state(X, 2, 41, amp=0.3, L=[2.0, 3.0])
+    u = u * (1.0 + 0.5 * (np.arange(u.shape[1]) % 4 == 0))[None, :, None]
+    du = torch.tensor(u.reshape(-1), dtype=torch.float64, device=cuda)
+    a = torch.empty_like(du)
+    op.Mult(du, a)
+    torch.cuda.synchronize()
+    assert rel(a.cpu().numpy(), orc.Mult(u)) <= 1e-12
