@@ -287,11 +287,11 @@ int prandtl_set_shape(prandtl_ctx *ctx, int kernel, int shape);
 /* Kernel algorithm of the flux-differencing RHS (no counterpart in the
  * reference; the operator is the same, DGSEMIntegrator.cpp:151-1196).  Every
  * 2-D and 3-D mesh runs k_rhs_l, one thread per tensor line.  Periodic
- * Cartesian boxes in 3-D, N = 2..4, have two settings: PRANDTL_ALGO_LINE (the
- * default at N = 2 and 3 and, with blending, at N = 4) runs the mixed form's
- * viscous kernel at N = 3 with its derivative contractions on the FP32
- * matrix cores (k_visc_mx) and has launch shape 0 only; PRANDTL_ALGO_TILE
- * runs k_visc and has the forced launch shapes.  Their FP64 results are the
+ * Cartesian boxes in 3-D, N = 2..4, have two settings that run the same
+ * kernels: PRANDTL_ALGO_LINE (the default at N = 2 and 3 and, with blending,
+ * at N = 4) has launch shape 0 only (both kernels in the mixed form at N = 3,
+ * else the RHS kernel), PRANDTL_ALGO_TILE the forced launch shapes.  Their
+ * results are the
  * same.  Every other context reports PRANDTL_ALGO_TILE, and
  * PRANDTL_ERR_UNSUPPORTED for PRANDTL_ALGO_LINE. */
 #define PRANDTL_ALGO_TILE 0

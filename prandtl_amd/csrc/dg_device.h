@@ -5,13 +5,15 @@
 //
 // Two kernels per RHS evaluation:
 //
-//  k_visc (parabolic only)  u -> BR1 lifting of the entropy variables,
+//  k_visc_l (dg_visc_lines.h: boxes, corrected mode) or k_visc (meshes,
+//  faithful mode, gradient output), parabolic only  u -> BR1 lifting of the entropy variables,
 //      EntropyGrad2PrimGrad, viscous flux, contravariant transform and the
 //      weak-form derivative sum D^ Fv of the volume term; writes the raw
 //      viscous volume sum (nv-1 per node) and the face-normal component of
 //      the viscous flux at every face node of the element (nv-1 per face
 //      node).  Restates DGSEMOperator.cpp:82-159, LiftingBR1.cpp:10-272 and
 //      DGSEMIntegrator.cpp:617-641,705-738 (and 435-549 for the face side).
+//      The volume sum holds this element's half of the viscous face terms.
 //
 //  k_rhs_l (dg_lines.h; k_rhs in 1-D)  the inviscid flux differencing,
 //      surface fluxes, modal indicator and subcell FV blending, plus the
@@ -113,8 +115,18 @@ struct KArgs {
     const int *skip;      // if set and nonzero, the launch does nothing (a finished device loop)
 };
 
+// A (N+1)x(N+1) derivative matrix M with M[N-a][N-m] = -M[a][m] in even-odd
+// form, H = NP/2 rows: e, o = (M[a][m] +- M[a][N-m]) / 2 at 4a + m, c the
+// middle column, r the middle row (odd NP).
+struct EvenOdd {
+    double e[16], o[16], c[4], r[4];
+};
+
 struct VArgs {
     Tables tab;
+    EvenOdd eD;           // D
+    double iw0;           // 1/w_0
+
     Geo geo;
     Phys phys;
     int quirks;
@@ -991,6 +1003,12 @@ __attribute__((amdgpu_waves_per_eu(VCfg<DIM, NP, FB>::WAVES))) k_visc(const VArg
     }
     __syncthreads();   // sW/sWN are dead from here; sFV reuses their storage
 
+    // this element's half of its face traces, which belongs to the face terms
+    // +-(1/w0) (Fv.n own + neighbour)/2 and goes into the volume sums (k_rhs_l
+    // adds the neighbour's half; a boundary side's flux is k_rhs_l's alone)
+    R own[NV - 1];
+#pragma unroll
+    for (int v = 0; v < NV - 1; v++) own[v] = 0;
     if (act) {
         R fl[DIM + 1][DIM];
         // volume viscous flux uses the stale node K-1 state (DGSEMIntegrator.cpp:620)
@@ -1035,10 +1053,18 @@ __attribute__((amdgpu_waves_per_eu(VCfg<DIM, NP, FB>::WAVES))) k_visc(const VArg
 #pragma unroll
                             for (int d = 1; d < DIM; d++) a = a + fl[v - 1][d] * nf[d];
                             dst[(v - 1) * NFP + l] = a;
+                            const int code = A.geo.fface[ef];
+                            const R h = ((code >> 1) & 7) != BC_PERIODIC ? R(0) : (R)(0.5 / A.tab.w[0]);
+                            own[v - 1] += ((code & 1) ? h : -h) * a;
                         }
                     } else {
+                        R h = (R)(0.5 / A.tab.w[0]) * (R)A.geo.nrm[c];
+                        if (OPEN && boundary_of(A.geo, e, c, side) != BC_PERIODIC) h = 0;
 #pragma unroll
-                        for (int v = 1; v < NV; v++) dst[(v - 1) * NFP + l] = fl[v - 1][c];
+                        for (int v = 1; v < NV; v++) {
+                            dst[(v - 1) * NFP + l] = fl[v - 1][c];
+                            own[v - 1] += (side ? h : -h) * fl[v - 1][c];
+                        }
                     }
                 }
             }
@@ -1063,7 +1089,7 @@ __attribute__((amdgpu_waves_per_eu(VCfg<DIM, NP, FB>::WAVES))) k_visc(const VArg
             }
         }
 #pragma unroll
-        for (int v = 0; v < NV - 1; v++) visc[v * NK + (size_t)e * K + n] = acc[v];
+        for (int v = 0; v < NV - 1; v++) visc[v * NK + (size_t)e * K + n] = acc[v] + own[v];
     }
 }
 

@@ -438,11 +438,28 @@ int rhs_only(prandtl_ctx *c, const double *y, double *out, hipStream_t s)
     PRANDTL_DISPATCH(launch_rhs, c, y, nullptr, out, 0, 0.0, 0.0, 0.0, s)
 }
 
+// Even-odd form of D.
+void even_odd(int Np, const double *D, EvenOdd &M)
+{
+    const int N = Np - 1, H = Np / 2;
+    std::memset(&M, 0, sizeof(M));
+    for (int a = 0; a < H; a++) {
+        for (int m = 0; m < H; m++) {
+            const double d = D[a * MAXNP + m], b = D[a * MAXNP + N - m];
+            M.e[4 * a + m] = 0.5 * (d + b);
+            M.o[4 * a + m] = 0.5 * (d - b);
+        }
+        if (Np & 1) M.c[a] = D[a * MAXNP + H];
+    }
+    if (Np & 1)
+        for (int m = 0; m < H; m++) M.r[m] = D[H * MAXNP + m];
+}
+
 bool shape_ok(const prandtl_ctx *c, int kernel, int shape)
 {
     if (kernel == PRANDTL_KERNEL_VISC)
         return c->prm.parabolic &&
-               (shape == 0 || (!c->geo.bcmask && !c->gen && !visc_mx_ok(c) && visc_shape_ok(c->dim, c->Np, shape)));
+               (shape == 0 || (!c->geo.bcmask && !c->gen && !visc_shape_fixed(c) && visc_shape_ok(c->dim, c->Np, shape)));
     if (kernel != PRANDTL_KERNEL_RHS) return false;
     if (shape == 0) return true;
     if (c->rhs_algo == PRANDTL_ALGO_LINE) return false;
@@ -665,6 +682,7 @@ int create_impl(const prandtl_mesh_desc *mesh, const prandtl_quad_mesh *qm, cons
     c->tab.Dh[N * MAXNP + N] -= 1.0 / w[N];
     c->tab.Dh2[0] += 1.0 / w[0];
     c->tab.Dh2[N * MAXNP + N] -= 1.0 / w[N];
+    even_odd(Np, c->tab.D, c->eD);
     // modal basis: 1-D shifted Legendre Vandermonde (ModalBasis.cpp:110-135)
     std::vector<double> V(Np * Np), Vi;
     for (int i = 0; i < Np; i++) {

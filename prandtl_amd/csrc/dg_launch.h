@@ -1,12 +1,11 @@
-// Host-side launch templates of k_visc and k_rhs and the context they read.
+// Host-side launch templates of the viscous and RHS kernels and the context they read.
 // Each (dimension, order) pair is instantiated in its own translation unit
 // (inst_*.hip, listed by PRANDTL_ORDERS) so the library builds in parallel.
 #pragma once
 #include <string>
 #include <vector>
 #include "dg_device.h"
-#include "dg_lines.h"
-#include "dg_visc_mx.h"
+#include "dg_visc_lines.h"
 
 using namespace prandtl;
 
@@ -15,6 +14,7 @@ struct prandtl_ctx {
     prandtl_mesh_desc mesh;
     prandtl_params prm;
     Tables tab;
+    EvenOdd eD;
     Geo geo;
     Phys phys;
     double *d_visc = nullptr, *d_fvf = nullptr, *d_alpha = nullptr, *d_eta = nullptr;
@@ -54,9 +54,9 @@ struct prandtl_ctx {
     int nattr = 0;
     double graph_dt = 0.0;        // value last copied to d_dt
     bool graph_dt_set = false;
-    int rhs_algo = 0;             // flux-differencing kernel: PRANDTL_ALGO_TILE (k_rhs) or _LINE (k_rhs_ln)
+    int rhs_algo = 0;             // PRANDTL_ALGO_TILE or _LINE (line_ok)
     int rhs_shape = 0;            // k_rhs launch shape (only shapes rhs_shape_ok accepts are set)
-    int visc_shape = 0;           // k_visc launch shape (visc_shape_ok)
+    int visc_shape = 0;           // k_visc / k_visc_l launch shape (visc_shape_ok)
     // device time loop (prandtl_run)
     LoopState *d_loop = nullptr;
     const int *skip = nullptr;    // set while launching the loop's stages
@@ -105,21 +105,37 @@ struct ProfScope {
     }
 };
 
+// k_visc in one launch shape (boxes in faithful mode, FP64).
 template <int DIM, int NP, int FB> void launch_visc_fb(prandtl_ctx *c, const VArgs &a, hipStream_t s)
 {
     using Cf = VCfg<DIM, NP, FB>;
     const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-    if (c->prm.precision == PRANDTL_MIXED)
-        hipLaunchKernelGGL((k_visc<DIM, NP, true, FB>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-    else hipLaunchKernelGGL((k_visc<DIM, NP, false, FB>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+    hipLaunchKernelGGL((k_visc<DIM, NP, false, FB>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
 }
+
+// k_visc_l in one launch shape.
+template <int DIM, int NP, int FB, bool OPEN> void launch_visc_l(prandtl_ctx *c, const VArgs &a, hipStream_t s)
+{
+    using Cf = VlCfg<DIM, NP, FB>;
+    const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
+    if (c->prm.precision == PRANDTL_MIXED)
+        hipLaunchKernelGGL((k_visc_l<DIM, NP, true, FB, OPEN>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+    else hipLaunchKernelGGL((k_visc_l<DIM, NP, false, FB, OPEN>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+}
+
+// A smaller workgroup for meshes too small for the natural one: with fewer
+// natural workgroups than CUs (256), one or two elements per workgroup spread
+// over more of them.  Euler right-hand sides, natural against this: 3-D N = 3
+// 512 elements 9.3 -> 8.0 us (2,197 elements 15.7 against 14.0, 4,096 18.6
+// against 18.7), N = 4 252 elements 10.8 -> 8.9, N = 2 125 elements 10.7 -> 8.5.
+constexpr int lines_small_fb(int DIM, int NP) { return DIM != 3 || NP > 6 ? 0 : NP <= 4 ? 64 : 128; }
 
 // Orders the general-geometry kernels are built for: 2-D N = 1..5, 3-D N = 2..4.
 constexpr bool gen_built(int DIM, int NP) { return DIM == 2 ? NP <= 6 : DIM == 3 && NP <= 5; }
 
-// The MFMA viscous kernel serves the mixed form of the line algorithm on
-// periodic 3-D boxes at N = 3.
-inline bool visc_mx_ok(const prandtl_ctx *c)
+// The mixed form of the line algorithm on periodic 3-D boxes at N = 3 has no
+// choice of viscous launch shape.
+inline bool visc_shape_fixed(const prandtl_ctx *c)
 {
     return c->rhs_algo == PRANDTL_ALGO_LINE && c->prm.precision == PRANDTL_MIXED && c->dim == 3 && c->Np == 4 &&
            !c->gen && !c->axi && c->geo.bcmask == 0;
@@ -128,19 +144,11 @@ inline bool visc_mx_ok(const prandtl_ctx *c)
 template <int DIM, int NP> int launch_visc_nd(prandtl_ctx *c, const double *y, double *grad, hipStream_t s)
 {
     VArgs a;
-    a.tab = c->tab; a.geo = c->geo; a.phys = c->phys;
+    a.tab = c->tab; a.eD = c->eD; a.iw0 = 1.0 / c->tab.w[0]; a.geo = c->geo; a.phys = c->phys;
     a.quirks = c->prm.quirks;
     a.y = y; a.visc = c->d_visc; a.fvf = c->d_fvf; a.grad = grad;
     a.skip = c->skip;
     ProfScope ps(c, s, 1);
-    if constexpr (DIM == 3 && NP == 4) {
-        if (visc_mx_ok(c)) {
-            using Mc = MxCfg<NP>;
-            const int nb = (c->NE + Mc::EPB - 1) / Mc::EPB;
-            hipLaunchKernelGGL((k_visc_mx<NP>), dim3(nb), dim3(Mc::BLOCK), 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_visc_mx launch");
-        }
-    }
     if constexpr (gen_built(DIM, NP)) {
         if (c->gen) {
             // quadrilateral or hexahedral mesh, natural shape
@@ -152,13 +160,40 @@ template <int DIM, int NP> int launch_visc_nd(prandtl_ctx *c, const double *y, d
             return hip_check(c, hipGetLastError(), "k_visc launch");
         }
     }
-    if (c->geo.bcmask) {
-        // boundary sides: the open variant, natural shape
+    if (!c->prm.quirks && !grad) {
+        constexpr int SM = lines_small_fb(DIM, NP);
+        const bool small = SM > 0 && c->NE < 256 * LnCfg<DIM, NP>::EPB;
+        if (c->geo.bcmask) {
+            if (small) launch_visc_l<DIM, NP, SM, true>(c, a, s);
+            else launch_visc_l<DIM, NP, 0, true>(c, a, s);
+        } else {
+            switch (c->visc_shape) {
+            case 1:
+                if constexpr (visc_shape_ok(DIM, NP, 1)) launch_visc_l<DIM, NP, 64, false>(c, a, s);
+                break;
+            case 2:
+                if constexpr (visc_shape_ok(DIM, NP, 2)) launch_visc_l<DIM, NP, 128, false>(c, a, s);
+                break;
+            case 3:
+                if constexpr (visc_shape_ok(DIM, NP, 3)) launch_visc_l<DIM, NP, 256, false>(c, a, s);
+                break;
+            default:
+                if (small) launch_visc_l<DIM, NP, SM, false>(c, a, s);
+                else launch_visc_l<DIM, NP, 0, false>(c, a, s);
+                break;
+            }
+        }
+        return hip_check(c, hipGetLastError(), "k_visc_l launch");
+    }
+    if (c->geo.bcmask || grad) {
+        // boundary sides, or the gradient output: natural shape
         using Cf = VCfg<DIM, NP, 0>;
-        const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-        if (c->prm.precision == PRANDTL_MIXED)
-            hipLaunchKernelGGL((k_visc<DIM, NP, true, 0, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-        else hipLaunchKernelGGL((k_visc<DIM, NP, false, 0, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+        const dim3 nb((c->NE + Cf::EPB - 1) / Cf::EPB), bl(Cf::BLOCK);
+        const bool mixed = c->prm.precision == PRANDTL_MIXED;
+        if (c->geo.bcmask && mixed) hipLaunchKernelGGL((k_visc<DIM, NP, true, 0, true>), nb, bl, 0, s, a);
+        else if (c->geo.bcmask) hipLaunchKernelGGL((k_visc<DIM, NP, false, 0, true>), nb, bl, 0, s, a);
+        else if (mixed) hipLaunchKernelGGL((k_visc<DIM, NP, true, 0>), nb, bl, 0, s, a);
+        else hipLaunchKernelGGL((k_visc<DIM, NP, false, 0>), nb, bl, 0, s, a);
         return hip_check(c, hipGetLastError(), "k_visc launch");
     }
     switch (c->visc_shape) {
@@ -193,8 +228,8 @@ inline bool line_ok(const prandtl_ctx *c)
     return line_built(c->dim, c->Np) && !c->gen && !c->axi && c->geo.bcmask == 0;
 }
 
-// The default there.  Both values run k_rhs_l; LINE adds k_visc_mx in the
-// mixed form at N = 3, TILE the forced launch shapes.
+// The default there.  Both values run the same kernels; TILE admits the forced
+// launch shapes.
 inline bool line_default(const prandtl_ctx *c)
 {
     return line_ok(c) && (c->Np <= 4 || c->prm.blending);
@@ -228,13 +263,6 @@ int launch_lines(prandtl_ctx *c, const KArgs &a, hipStream_t s)
     hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, double, FB, OPEN, GEN>), nb, bl, 0, s, a);
     return hip_check(c, hipGetLastError(), "k_rhs_l launch");
 }
-
-// A smaller workgroup for meshes too small for the natural one: with fewer
-// natural workgroups than CUs (256), one or two elements per workgroup spread
-// over more of them.  Euler right-hand sides, natural against this: 3-D N = 3
-// 512 elements 9.3 -> 8.0 us (2,197 elements 15.7 against 14.0, 4,096 18.6
-// against 18.7), N = 4 252 elements 10.8 -> 8.9, N = 2 125 elements 10.7 -> 8.5.
-constexpr int lines_small_fb(int DIM, int NP) { return DIM != 3 || NP > 6 ? 0 : NP <= 4 ? 64 : 128; }
 
 template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN>
 int launch_lines_sized(prandtl_ctx *c, const KArgs &a, hipStream_t s)

@@ -124,6 +124,45 @@ template <int DIM, int NP, int FB = 0> struct LnCfg {
 // LDS reads cost more (2-D N = 3 slip-wall and mesh kernels 3-4% slower).
 constexpr bool lines_ltab(int DIM, int NP, bool BLEND) { return NP >= 6 || (DIM == 3 && NP >= 4 && BLEND); }
 
+// Which line a thread holds: element el of the workgroup, direction r, line l
+// with the other indices la, lb (increasing direction), rem = r NFP + l; base
+// and stride give its nodes' numbers, slots() their LDS slots.  NP = 8: a wave
+// is one direction, so r is scalar.
+template <int DIM, int NP, int FB> struct LinePos {
+    using C = LnCfg<DIM, NP, FB>;
+    int el, r, l, rem, la, lb, base, stride;
+    __device__ __forceinline__ explicit LinePos(int t)
+    {
+        constexpr int NFP = C::NFP, TE = C::TE;
+        if constexpr (C::HALF) {
+            const int h = t >> 5;
+            r = h % 3;
+            el = 2 * (h / 3) + ((t >> 4) & 1);
+            l = t & 15;
+            rem = r * NFP + l;
+        } else {
+            el = C::EPB == 1 ? 0 : t / TE;
+            rem = t - el * TE;
+            r = DIM == 1 ? 0 : rem / NFP;
+            if constexpr (NFP == 64 && C::EPB == 1) r = __builtin_amdgcn_readfirstlane(r);
+            l = rem - r * NFP;
+        }
+        la = DIM == 3 ? l % NP : l;
+        lb = DIM == 3 ? l / NP : 0;
+        base = DIM == 1 ? 0 : r == 0 ? l * NP : (DIM == 3 && r == 1 ? lb * NP * NP + la : l);
+        stride = r == 0 ? 1 : (r == 1 ? NP : NP * NP);
+    }
+    __device__ __forceinline__ void slots(int *ls) const
+    {
+#pragma unroll
+        for (int m = 0; m < NP; m++) {
+            if constexpr (DIM == 1) ls[m] = m;
+            else if constexpr (DIM == 2) ls[m] = r == 0 ? lines_slot<DIM, NP>(m, la, 0) : lines_slot<DIM, NP>(la, m, 0);
+            else ls[m] = lines_slot<DIM, NP>(r == 0 ? m : la, r == 1 ? m : (r == 0 ? la : lb), r == 2 ? m : lb);
+        }
+    }
+};
+
 // LDS of one tile (EPB elements).
 template <int DIM, int NP, bool BLEND, int FB, bool GEN, bool AXI> struct LineSmem {
     using C = LnCfg<DIM, NP, FB>;
@@ -249,35 +288,12 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
     const bool quirk3d = A.quirks != 0;
     const double lam_old = (t == 0) ? A.lam[slot] : 0.0;
 
-    // this thread's line: element el, direction r, line l with the other
-    // indices la, lb (increasing direction).  NP = 8: a wave is one direction,
-    // so r is scalar
-    int el, r, l, rem;
-    if constexpr (C::HALF) {
-        const int h = t >> 5;
-        r = h % 3;
-        el = 2 * (h / 3) + ((t >> 4) & 1);
-        l = t & 15;
-        rem = r * NFP + l;
-    } else {
-        el = EPB == 1 ? 0 : t / TE;
-        rem = t - el * TE;
-        r = DIM == 1 ? 0 : rem / NFP;
-        if constexpr (NFP == 64 && EPB == 1) r = __builtin_amdgcn_readfirstlane(r);
-        l = rem - r * NFP;
-    }
-    const int la = DIM == 3 ? l % NP : l, lb = DIM == 3 ? l / NP : 0;
+    const LinePos<DIM, NP, FB> L(t);
+    const int el = L.el, r = L.r, l = L.l, rem = L.rem, la = L.la, lb = L.lb, base = L.base, stride = L.stride;
     const int e = ebase + el;
     const bool lact = (el < EPB) && (rem < TE) && (e < NE);
-    const int base = DIM == 1 ? 0 : r == 0 ? l * NP : (DIM == 3 && r == 1 ? lb * NP * NP + la : l);
-    const int stride = r == 0 ? 1 : (r == 1 ? NP : NP * NP);
     int ls[NP];
-#pragma unroll
-    for (int m = 0; m < NP; m++) {
-        if constexpr (DIM == 1) ls[m] = m;
-        else if constexpr (DIM == 2) ls[m] = r == 0 ? lines_slot<DIM, NP>(m, la, 0) : lines_slot<DIM, NP>(la, m, 0);
-        else ls[m] = lines_slot<DIM, NP>(r == 0 ? m : la, r == 1 ? m : (r == 0 ? la : lb), r == 2 ? m : lb);
-    }
+    L.slots(ls);
 
     // ---- start loads: the nodes first, then the traces at the line's ends.
     // Loads complete in issue order, so the node phase waits for its own
@@ -312,7 +328,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
     double pt[2][NV];       // neighbour states; on a boundary side this element's own face node
     int bt[2] = {BC_PERIODIC, BC_PERIODIC};
     double nv[GEN ? 2 : 1][DIM];   // GEN: the end points' normals, outward of the face's first element
-    VT fto[2][NV - 1], ftn[2][NV - 1];
+    VT ftn[2][NV - 1];
 #pragma unroll
     for (int side = 0; side < 2; side++) {
         size_t g = 0;
@@ -342,14 +358,15 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
             }
         }
         if constexpr (DIM > 1 && !AXI) {
-            // viscous face traces of this side and of the neighbour; without
-            // viscous terms they are read from the state array and discarded
+            // the neighbour's viscous face trace (this element's own is in
+            // k_visc's volume term); without viscous terms it is read from
+            // the state array and discarded.  On a boundary side: this
+            // element's own trace
             const bool vact = A.parabolic && lact;
             const VT *fv = A.parabolic ? static_cast<const VT *>(A.fvf) : reinterpret_cast<const VT *>(A.y);
-            size_t oo = 0, on = 0;
+            size_t on = 0;
             if (vact) {
                 const size_t ef = (size_t)e * 2 * DIM + 2 * r + side;
-                oo = ef * (NV - 1) * NFP + l;
                 if constexpr (GEN) {
                     if (bt[side] == BC_PERIODIC) {
                         const int nf = A.geo.fnf[ef];
@@ -358,15 +375,17 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                         if constexpr (DIM == 2) l2 = (nf & 1) ? NP - 1 - l : l;
                         else l2 = face_point_3<NP>(gn[side] - (int)(fid / 6) * K, (int)(fid % 6) >> 1);
                         on = fid * (NV - 1) * NFP + l2;
+                    } else {
+                        on = ef * (NV - 1) * NFP + l;
                     }
                 } else {
-                    on = ((size_t)en * 2 * DIM + 2 * r + 1 - side) * (NV - 1) * NFP + l;
+                    const bool bnd = OPEN && bt[side] != BC_PERIODIC;
+                    on = (bnd ? ef : (size_t)en * 2 * DIM + 2 * r + 1 - side) * (NV - 1) * NFP + l;
                 }
             }
 #pragma unroll
             for (int v = 0; v < NV - 1; v++) {
-                const VT a = fv[oo + v * NFP], b = fv[on + v * NFP];
-                fto[side][v] = vact ? a : VT(0);
+                const VT b = fv[on + v * NFP];
                 ftn[side][v] = vact ? b : VT(0);
             }
         }
@@ -517,7 +536,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
 #pragma unroll
                         for (int d = 1; d < DIM; d++) n2 = n2 + nn[d] * nn[d];
 #pragma unroll
-                        for (int v = 1; v < NV; v++) fn[v] = GEN ? (double)fto[side][v - 1] : (double)fto[side][v - 1] * (side ? nr : -nr);
+                        for (int v = 1; v < NV; v++) fn[v] = GEN ? (double)ftn[side][v - 1] : (double)ftn[side][v - 1] * (side ? nr : -nr);
                         if (bt[side] == BC_NOSLIP) {
                             double en = bs[0] * fn[1];
 #pragma unroll
@@ -570,10 +589,11 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
             }
             if constexpr (DIM > 1 && !AXI) {
                 if (A.parabolic) {
-                    // the mean of the two sides' traces Fv.n (boxes: per unit normal)
+                    // the neighbour's half of the mean of the two sides' traces
+                    // Fv.n (boxes: per unit normal)
                     const double hn = GEN ? 0.5 : 0.5 * nr;
 #pragma unroll
-                    for (int v = 1; v < NV; v++) F[v] -= ((double)fto[side][v - 1] + (double)ftn[side][v - 1]) * hn;
+                    for (int v = 1; v < NV; v++) F[v] -= (double)ftn[side][v - 1] * hn;
                 }
             }
             const double sg = own ? iw0 : -iw0;
