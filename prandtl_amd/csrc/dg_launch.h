@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 #include "dg_device.h"
+#include "dg_points.h"
 #include "dg_visc_lines.h"
 
 using namespace prandtl;
@@ -264,9 +265,41 @@ int launch_lines(prandtl_ctx *c, const KArgs &a, hipStream_t s)
     return hip_check(c, hipGetLastError(), "k_rhs_l launch");
 }
 
+// Whether a mesh takes k_rhs_p instead of k_rhs_l: by the waves its node
+// threads fill (1024 are one per SIMD).  The longer a line's chain (pairs,
+// mesh metrics, subcell fluxes), the later its line threads win.  us per
+// right-hand side, line / node threads, below and above the limit:
+//   2-D N = 2 3,906 quadrilaterals 11.3 / 9.6, 6,480 boxes 7.6 / 8.6; N = 3 3,906
+//   blended 10.2 / 9.1, 4,692 8.2 / 9.2; N = 4 1,640 8.6 / 8.1, 2,162 8.7 / 9.6,
+//   blended 1,640 13.5 / 9.1, 2,756 13.7 / 11.1, 4,692 14.5 / 15.9; N = 5 2,162
+//   quadrilaterals 15.1 / 12.6, 2,756 15.4 / 15.7;
+//   3-D N = 2 blended 336 11.1 / 10.3, 1,716 11.6 / 13.2 (without blending no gain);
+//   N = 3 120 hexahedra 10.4 / 8.2, 720 10.0 / 10.5; N = 4 210 10.6 / 8.6, 336
+//   hexahedra 12.8 / 16.1; N = 5 210 14.0 / 11.2, 336 14.4 / 18.1.
+template <int DIM, int NP, bool BLEND, bool GEN> constexpr int points_waves()
+{
+    if (DIM == 2) return NP == 2 ? 768 : NP == 3 ? 1792 : NP == 4 ? 2048 : NP == 5 && !BLEND && !GEN ? 1792 : 3072;
+    return NP == 3 ? (BLEND ? 512 : 0) : NP == 4 ? 1024 : NP == 5 ? 1536 : 2560;
+}
+
+template <int DIM, int NP, bool BLEND, bool GEN> bool points_ok(const prandtl_ctx *c)
+{
+    using Pc = PtCfg<DIM, NP>;
+    if (c->axi || (c->prm.parabolic && (c->prm.quirks || c->prm.precision == PRANDTL_MIXED))) return false;
+    return (long long)(c->NE + Pc::EPB - 1) / Pc::EPB * (Pc::BLOCK / 64) <= points_waves<DIM, NP, BLEND, GEN>();
+}
+
 template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN>
 int launch_lines_sized(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
+    if constexpr (points_built(DIM, NP)) {
+        if (points_ok<DIM, NP, BLEND, GEN>(c)) {
+            using Pc = PtCfg<DIM, NP>;
+            hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, OPEN, GEN>), dim3((c->NE + Pc::EPB - 1) / Pc::EPB),
+                               dim3(Pc::BLOCK), 0, s, a);
+            return hip_check(c, hipGetLastError(), "k_rhs_p launch");
+        }
+    }
     constexpr int SM = lines_small_fb(DIM, NP);
     if constexpr (SM > 0) {
         if (c->NE < 256 * LnCfg<DIM, NP>::EPB) return launch_lines<DIM, NP, BLEND, SM, OPEN, GEN>(c, a, s);
