@@ -154,10 +154,12 @@ template <int DIM, int NP> int launch_visc_nd(prandtl_ctx *c, const double *y, d
         if (c->gen) {
             // quadrilateral or hexahedral mesh, natural shape
             using Cf = VCfg<DIM, NP, 0>;
-            const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-            if (c->prm.precision == PRANDTL_MIXED)
-                hipLaunchKernelGGL((k_visc<DIM, NP, true, 0, false, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-            else hipLaunchKernelGGL((k_visc<DIM, NP, false, 0, false, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
+            const dim3 nb((c->NE + Cf::EPB - 1) / Cf::EPB), bl(Cf::BLOCK);
+            const bool mixed = c->prm.precision == PRANDTL_MIXED, red = !c->prm.quirks && !grad;
+            if (mixed && red) hipLaunchKernelGGL((k_visc<DIM, NP, true, 0, false, true, true>), nb, bl, 0, s, a);
+            else if (mixed) hipLaunchKernelGGL((k_visc<DIM, NP, true, 0, false, true>), nb, bl, 0, s, a);
+            else if (red) hipLaunchKernelGGL((k_visc<DIM, NP, false, 0, false, true, true>), nb, bl, 0, s, a);
+            else hipLaunchKernelGGL((k_visc<DIM, NP, false, 0, false, true>), nb, bl, 0, s, a);
             return hip_check(c, hipGetLastError(), "k_visc launch");
         }
     }

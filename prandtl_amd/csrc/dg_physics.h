@@ -515,8 +515,9 @@ __device__ __forceinline__ double boundary_flux(int type, int r, double ns, doub
     return (q1.lam < q2.lam) ? q2.lam : q1.lam;
 }
 
-// Conserv2Entropy, BasicOperations.cpp:81-104 (beta = rho/p)
-template <int DIM>
+// Conserv2Entropy, BasicOperations.cpp:81-104 (beta = rho/p); FIRST = false:
+// all but w[0], which alone needs logarithms
+template <int DIM, bool FIRST = true>
 __device__ __forceinline__ void cons2entropy(const double *s, const Phys &P, double *w)
 {
     const double r = rcp_nr(s[0]);
@@ -531,8 +532,10 @@ __device__ __forceinline__ void cons2entropy(const double *s, const Phys &P, dou
     const double beta = s[0] * rcp_nr(p);
     // log(p rho^-gamma) as log p - gamma log rho: two logs instead of a log
     // and a pow (rounding-level difference)
-    const double sent = log(p) - P.gamma * log(s[0]);
-    w[0] = (P.gamma - sent) * P.gm1i - beta * v_sq;
+    if constexpr (FIRST) {
+        const double sent = log(p) - P.gamma * log(s[0]);
+        w[0] = (P.gamma - sent) * P.gm1i - beta * v_sq;
+    }
 #pragma unroll
     for (int d = 0; d < DIM; d++) w[1 + d] = beta * vel[d];
     w[DIM + 1] = -beta;
@@ -612,6 +615,30 @@ __device__ __forceinline__ void entgrad2primgrad(const R *s, R gm1, R gm1i, bool
     }
     g[0] = s[0] * g0 - gL * (KE - p * gm1i) + rp * mdot;
     g[DIM + 1] = pr * (g[0] + p * gL);
+}
+
+// EntropyGrad2PrimGrad in corrected mode, as far as viscous_flux with the same
+// state needs it: grad v = T (grad(beta v) - v grad beta) and, in the place of
+// the pressure's, rho grad T = rho T^2 grad(-beta) with a density gradient of
+// zero: the density gradient, which the first entropy variable's is for,
+// drops out of the heat flux.
+template <int DIM, typename R>
+__device__ __forceinline__ void entgrad2velgrad(const R *s, R gm1, R *g)
+{
+    const R half = 0.5;
+    const R r = rcp_nr(s[0]);
+    R vel[DIM], vv = 0;
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        vel[d] = s[1 + d] * r;
+        vv = (d == 0) ? vel[d] * vel[d] : vv + vel[d] * vel[d];
+    }
+    const R p = gm1 * (s[DIM + 1] - s[0] * (half * vv));
+    const R T = p * r, gL = g[DIM + 1];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) g[1 + d] = T * (g[1 + d] + vel[d] * gL);
+    g[0] = 0;
+    g[DIM + 1] = p * T * gL;
 }
 
 // NavierStokesFlux::ComputeViscousFlux (NavierStokesFlux.cpp:12-90), mu_bulk =
