@@ -60,6 +60,8 @@ struct prandtl_ctx {
     int visc_shape = 0;           // k_visc / k_visc_l launch shape (visc_shape_ok)
     // device time loop (prandtl_run)
     LoopState *d_loop = nullptr;
+    LoopState *h_loop = nullptr;            // pinned, two snapshots
+    hipEvent_t loop_ev[2] = {nullptr, nullptr};
     const int *skip = nullptr;    // set while launching the loop's stages
 };
 
