@@ -1,5 +1,5 @@
 // Device side of the DGSEM RHS (gfx950): tables and arguments, launch shapes,
-// mesh and index helpers, the 1-D kernel k_rhs and the viscous kernel k_visc.
+// mesh and index helpers and the viscous kernel k_visc.
 // Included by the library's host translation unit and by the per-order
 // instantiation units.
 //
@@ -15,7 +15,8 @@
 //      DGSEMIntegrator.cpp:617-641,705-738 (and 435-549 for the face side).
 //      The volume sum holds this element's half of the viscous face terms.
 //
-//  k_rhs_l (dg_lines.h; k_rhs in 1-D)  the inviscid flux differencing,
+//  k_rhs_l (dg_lines.h; dg_points.h's k_rhs_p in 1-D and on small meshes)
+//      the inviscid flux differencing,
 //      surface fluxes, modal indicator and subcell FV blending, plus the
 //      viscous volume/face terms from k_visc, then either writes the RHS
 //      (Operator::Mult) or the RK3 stage combination.
@@ -55,7 +56,6 @@ struct Tables {
     double Dh[MAXNP * MAXNP];   // D + E            (lines 71-74, un-transposed)
     double Dh2[MAXNP * MAXNP];  // 2D + E           (lines 76-80, un-transposed)
     double V1i[MAXNP * MAXNP];  // inverse 1-D shifted-Legendre Vandermonde
-    double fvs[MAXNP];          // 1/(J w_i)            (line 1046)
     double w[MAXNP];            // LGL weights on [0,1]
     double x[MAXNP];            // LGL nodes on [0,1]
     double subn[3][MAXNP];      // subcell normal magnitude per interface (1199-1304)
@@ -201,14 +201,6 @@ template <int NP> __device__ __forceinline__ int pair_index(int a, int b)
     return a * NP - (a * (a + 1)) / 2 + (b - a - 1);
 }
 
-template <int NP> __device__ __forceinline__ void pair_ab(int p, int &a, int &b)
-{
-    a = 0;
-    int rem = p;
-    while (rem >= NP - 1 - a) { rem -= NP - 1 - a; a++; }
-    b = a + 1 + rem;
-}
-
 __device__ __forceinline__ int xcd_remap(int bid, int nb)
 {
     // blocks are dispatched round-robin over the 8 XCDs; give each XCD a
@@ -259,14 +251,6 @@ __device__ __forceinline__ double step_dt(const KArgs &A)
     return dt;
 }
 
-__device__ __forceinline__ int neighbor(const Geo &g, int e, int r, int side)
-{
-    int idx[3];
-    box_index(g, e, idx);
-    idx[r] = side ? (idx[r] + 1 == g.n[r] ? 0 : idx[r] + 1) : (idx[r] == 0 ? g.n[r] - 1 : idx[r] - 1);
-    return (idx[2] * g.n[1] + idx[1]) * g.n[0] + idx[0];
-}
-
 // a, b or c for r = 0, 1, 2 where r differs between the lanes of a wave:
 // the three values pass through an empty asm first, so the choice is between
 // values, not a load through a selected address of the argument struct
@@ -276,8 +260,9 @@ __device__ __forceinline__ double lane_pick3(double a, double b, double c, int r
     return r == 0 ? a : r == 1 ? b : c;
 }
 
-// neighbor() for callers whose direction r differs between the lanes of a
-// wave (one thread per line or per face point of several directions).
+// The element beside e's face (r, side), periodic, for callers whose direction
+// r differs between the lanes of a wave (one thread per line or per face point
+// of several directions).
 // Indexing the argument struct with a per-lane r is a vector load from
 // argument memory that the thread waits for before its state loads can
 // issue; so is a select between the three fields, which the compiler turns
@@ -468,267 +453,6 @@ template <int NP> __device__ __forceinline__ int face_point_3(int node, int r)
 {
     const int i = node % NP, j = (node / NP) % NP, k = node / (NP * NP);
     return r == 0 ? j + NP * k : (r == 1 ? i + NP * k : i + NP * j);
-}
-
-// ---------------------------------------------------------------------------
-// k_rhs: 1-D boxes (Euler)
-// ---------------------------------------------------------------------------
-// A workgroup's threads take the elements' two-point fluxes as jobs: one node
-// per thread in the node phases, then surface points, then symmetric volume
-// pairs and subcell interfaces through LDS, summed per node in the
-// reference's order.  A 1-D mesh has one line per element, so a thread per
-// line (k_rhs_l) would leave a mesh of a few hundred elements with a handful of
-// waves and all of a line's fluxes in sequence: 128 elements with a shock, 32
-// steps of the device loop 1,560 us against 1,130 here.
-template <int NP, bool BLEND> struct R1Cfg {
-    static constexpr int NPAIR = NP * (NP - 1) / 2;
-    static constexpr int NFV = BLEND ? NP - 1 : 0;
-    static constexpr int JOBS = NPAIR + NFV;
-    static constexpr int WORK = cmx(NP, cmx(JOBS, 2));
-    static constexpr int EPB = cmx(1, 256 / WORK);
-    static constexpr int BLOCK = r64(EPB * WORK) > 512 ? 512 : r64(EPB * WORK);
-    static_assert(EPB * NP <= BLOCK, "one node per thread");
-};
-
-template <int NP, bool BLEND, bool OPEN>
-__global__ void __launch_bounds__((R1Cfg<NP, BLEND>::BLOCK))
-__attribute__((amdgpu_waves_per_eu(3))) k_rhs(const KArgs A)
-{
-    using C = R1Cfg<NP, BLEND>;
-    constexpr int NV = 3, NPAIR = C::NPAIR, NFV = C::NFV, JOBS = C::JOBS, EPB = C::EPB, BLOCK = C::BLOCK;
-    constexpr int NQ = BLEND ? 4 : 2;   // v, beta, (1/beta, lambda)
-    constexpr int FF = cmx(cmx(JOBS, 2), BLEND ? (4 * NP + NV - 1) / NV : 1);
-    static_assert(!BLEND || 4 * NP <= NV * FF, "indicator scratch fits the flux buffer");
-    __shared__ double sDh2[NP * NP], sV1i[BLEND ? NP * NP : 1], sFvs[NP], sSub[NP];
-    __shared__ double sU[EPB][NV][NP], sQ[EPB][NQ][NP];
-    __shared__ double sF[EPB][NV][FF];   // surface contributions, then the pair and subcell fluxes
-    __shared__ double sAl[EPB], sRed[(BLOCK + 63) / 64];
-
-    if (A.skip && *A.skip) return;   // uniform: before any barrier
-    const int t = threadIdx.x;
-    // the operator's tables, one entry per thread, loaded together and first
-    // (indices clamped, so every lane loads and no load waits for another);
-    // they go to LDS once the prologue's loads are in flight
-    static_assert(NP * NP <= BLOCK, "one table entry per thread");
-    const int tq = t < NP * NP ? t : 0, tf = t < NP ? t : 0;
-    const double tDh2 = A.tab.Dh2[(tq / NP) * MAXNP + tq % NP];
-    const double tV1i = BLEND ? A.tab.V1i[(tq / NP) * MAXNP + tq % NP] : 0.0;
-    const double tFvs = A.tab.fvs[tf], tSub = A.tab.subn[0][tf];
-
-    const Phys &P = A.phys;
-    const int NE = A.geo.NE;
-    const size_t NK = (size_t)NE * NP;
-    const int tile = xcd_remap(blockIdx.x, gridDim.x);
-    const int ebase = tile * EPB;
-    const int el = t / NP, n = t - el * NP;
-    const int e = ebase + el;
-    const bool act = (el < EPB) && (e < NE);
-    const double dt = step_dt(A);
-    const double lam_old = (t == 0) ? A.lam[blockIdx.x] : 0.0;
-    double ys[NV];
-    if (act)
-#pragma unroll
-        for (int v = 0; v < NV; v++) ys[v] = A.y[v * NK + (size_t)e * NP + n];
-    if (t < NP * NP) {
-        sDh2[t] = tDh2;
-        if (BLEND) sV1i[t] = tV1i;
-    }
-    if (t < NP) { sFvs[t] = tFvs; sSub[t] = tSub; }
-
-    // ---- node phase: state and per-node flux quantities into LDS ----
-    double lam = 0.0;
-    if (act) {
-#pragma unroll
-        for (int v = 0; v < NV; v++) sU[el][v][n] = ys[v];
-        const NodeQ<1> q = node_quants<1>(ys, P);
-        sQ[el][0][n] = q.v[0];
-        sQ[el][1][n] = q.beta;
-        if constexpr (BLEND) {
-            sQ[el][2][n] = q.ibeta;
-            sQ[el][3][n] = q.lam;
-        }
-        lam = (q.lam == q.lam) ? q.lam : 0.0;
-    }
-    __syncthreads();
-
-    // ---- modal indicator and blending coefficient (element-local) ----
-    if constexpr (BLEND) {
-        double *sX = &sF[0][0][0];
-        double *sM = sX + EPB * NP, *sE1 = sX + 2 * EPB * NP, *sE2 = sX + 3 * EPB * NP;
-        if (act) {
-            // rho * ComputePressure(state) with V /= rho (BasicOperations.cpp:31-37)
-            const double v = ys[1] * (1.0 / ys[0]);
-            sX[el * NP + n] = ys[0] * (P.gm1 * (ys[2] - 0.5 * ys[0] * (v * v)));
-        }
-        __syncthreads();
-        if (act) {
-            double s = 0.0;
-#pragma unroll
-            for (int i = 0; i < NP; i++)
-                s = (i == 0) ? sV1i[n * NP + i] * sX[el * NP + i] : s + sV1i[n * NP + i] * sX[el * NP + i];
-            // modal energies: all modes, modes of degree <= N-1 and <= N-2
-            // (PerssonPeraireIndicator.cpp:38-52), summed by a binary tree
-            const double e2 = s * s;
-            sM[el * NP + n] = e2;
-            sE1[el * NP + n] = n <= NP - 2 ? e2 : 0.0;
-            sE2[el * NP + n] = n <= NP - 3 ? e2 : 0.0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int h = pow2_at_least(NP) / 2; h >= 1; h >>= 1) {
-            if (act && n < h && n + h < NP) {
-                const int i0 = el * NP + n;
-                sM[i0] += sM[i0 + h];
-                sE1[i0] += sE1[i0 + h];
-                sE2[i0] += sE2[i0 + h];
-            }
-            __syncthreads();
-        }
-        if (act && n == 0) {
-            const double mm = sM[el * NP], m1 = sE1[el * NP], m2 = sE2[el * NP];
-            double eta = 1.0 - m1 / mm;
-            const double eta2 = 1.0 - m2 / m1;
-            eta = (eta < eta2) ? eta2 : eta;
-            // DGSEMOperator.cpp:67-77, sharpness 9.21024 (DGSEMOperator.hpp:50)
-            double al = 1.0 / (1.0 + exp(-9.21024 * (eta - P.thresh) / P.thresh));
-            if (al < P.alpha_min) al = 0.0;
-            else if (al > 1.0 - P.alpha_min) al = 1.0;
-            al = (P.alpha_max < al) ? P.alpha_max : al;
-            sAl[el] = al;
-            A.alpha[e] = al;
-            A.eta[e] = eta;
-        }
-        __syncthreads();
-    }
-    const double alpha_e = (BLEND && act) ? sAl[el] : 0.0;
-
-    // ---- the element's two surface points (elem1 = low side, normal +e_x),
-    // signed contribution for this element ----
-    const double nr = A.geo.nrm[0];
-    for (int jf = t; jf < EPB * 2; jf += BLOCK) {
-        const int ej = jf >> 1, side = jf & 1;
-        const int eo = ebase + ej;
-        if (eo >= NE) continue;
-        const int no = side ? NP - 1 : 0;
-        const int en = neighbor_lane(A.geo, eo, 0, side);
-        double so[NV], pn[NV], F[NV];
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            pn[v] = A.y[v * NK + (size_t)en * NP + (side ? 0 : NP - 1)];
-            so[v] = sU[ej][v][no];
-        }
-        if constexpr (OPEN) {
-            // boundary point: -F_b for the outward normal at the interior
-            // node (BdrFaceIntegrator.cpp:61-123, applied after the interior
-            // faces by DGSEMNonlinearForm.cpp:776-826); its wave speed joins
-            // the running maximum (DGSEMOperator.cpp:585-589)
-            const int bt = boundary_of(A.geo, eo, 0, side);
-            if (bt != BC_PERIODIC) {
-                double bs[5];
-#pragma unroll
-                for (int v = 0; v < 5; v++) bs[v] = A.geo.bcs[side * 5 + v];
-                const double lb = boundary_flux<1>(bt, 0, side ? nr : -nr, nr, so, bs, P, false, F);
-                lam = (lam < lb) ? lb : lam;
-#pragma unroll
-                for (int v = 0; v < NV; v++) sF[ej][v][side] = -F[v];
-                continue;
-            }
-        }
-        double s1[NV], s2[NV];
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            s1[v] = side ? so[v] : pn[v];
-            s2[v] = side ? pn[v] : so[v];
-        }
-        const NodeQ<1> q1 = node_quants<1>(s1, P), q2 = node_quants<1>(s2, P);
-        if (A.ec) ec_flux<1, false>(&nr, nr, q1, q2, P, false, F);
-        else ec_flux<1, true>(&nr, nr, q1, q2, P, false, F);
-#pragma unroll
-        for (int v = 0; v < NV; v++) sF[ej][v][side] = side ? -F[v] : F[v];
-    }
-    block_lam_max<BLOCK>(lam, lam_old, A.lam, sRed, blockIdx.x);
-    __syncthreads();
-    double accS[NV], accV[NV], accF[NV];
-#pragma unroll
-    for (int v = 0; v < NV; v++) {
-        accS[v] = accV[v] = accF[v] = 0.0;
-        if (act && n == 0) accS[v] += A.geo.aface * sF[el][v][0];
-        if (act && n == NP - 1) accS[v] += A.geo.aface * sF[el][v][1];
-    }
-    __syncthreads();
-
-    // ---- symmetric volume pairs (a < b) and subcell FV interfaces ----
-    for (int j = t; j < EPB * JOBS; j += BLOCK) {
-        // pairs of all elements first, then the interfaces
-        const bool pair = j < EPB * NPAIR;
-        const int jj = pair ? j : j - EPB * NPAIR;
-        const int ej = pair ? jj / NPAIR : jj / cmx(NFV, 1);
-        if (ebase + ej >= NE) continue;
-        double F[NV];
-        if (pair) {
-            const int p = jj - ej * NPAIR;
-            int a, b;
-            pair_ab<NP>(p, a, b);
-            NodeQ<1> qa, qb;
-            qa.rho = sU[ej][0][a]; qb.rho = sU[ej][0][b];
-            qa.v[0] = sQ[ej][0][a]; qb.v[0] = sQ[ej][0][b];
-            qa.beta = sQ[ej][1][a]; qb.beta = sQ[ej][1][b];
-            ec_flux<1, false>(&nr, nr, qa, qb, P, false, F);
-#pragma unroll
-            for (int v = 0; v < NV; v++) sF[ej][v][p] = F[v];
-        } else if constexpr (BLEND) {
-            const int i = jj - ej * NFV;
-            if (!(sAl[ej] > 0.0)) {
-#pragma unroll
-                for (int v = 0; v < NV; v++) sF[ej][v][NPAIR + i] = 0.0;
-                continue;
-            }
-            NodeQ<1> qa, qb;
-            qa.rho = sU[ej][0][i]; qb.rho = sU[ej][0][i + 1];
-            qa.v[0] = sQ[ej][0][i]; qb.v[0] = sQ[ej][0][i + 1];
-            qa.beta = sQ[ej][1][i]; qb.beta = sQ[ej][1][i + 1];
-            qa.ibeta = sQ[ej][NQ - 2][i]; qb.ibeta = sQ[ej][NQ - 2][i + 1];
-            qa.lam = sQ[ej][NQ - 1][i]; qb.lam = sQ[ej][NQ - 1][i + 1];
-            ec_flux<1, true>(&sSub[i], sSub[i], qa, qb, P, false, F);
-#pragma unroll
-            for (int v = 0; v < NV; v++) sF[ej][v][NPAIR + i] = F[v];
-        }
-    }
-    __syncthreads();
-    if (!act) return;   // no barrier follows
-#pragma unroll
-    for (int m = 0; m < NP; m++) {
-        if (m == n) continue;
-        const double dm = sDh2[n * NP + m];
-        const int p = m < n ? pair_index<NP>(m, n) : pair_index<NP>(n, m);
-#pragma unroll
-        for (int v = 0; v < NV; v++) accV[v] += dm * sF[el][v][p];
-    }
-    if (BLEND && alpha_e > 0.0) {
-        const double fvs = sFvs[n];
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            const double lo = n > 0 ? sF[el][v][NPAIR + n - 1] : 0.0;
-            const double hi = n < NP - 1 ? sF[el][v][NPAIR + n] : 0.0;
-            accF[v] = (lo - hi) * fvs;
-        }
-    }
-
-    // ---- assemble, stage update, store ----
-#pragma unroll
-    for (int v = 0; v < NV; v++) {
-        double vol = -accV[v];
-        if (BLEND) vol *= (1.0 - alpha_e);
-        vol *= A.geo.invJ;
-        const double tot = ((BLEND && alpha_e > 0.0) ? accF[v] * alpha_e + vol : vol) + accS[v];
-        const size_t gi = v * NK + (size_t)e * NP + n;
-        const double yv = sU[el][v][n];
-        double o;
-        if (A.mode == 0) o = tot;
-        else if (A.mode == 1) o = yv + dt * tot;
-        else o = A.c0 * A.u0[gi] + A.c1 * (yv + dt * tot);
-        A.out[gi] = o;
-    }
 }
 
 // ---------------------------------------------------------------------------

@@ -3,7 +3,7 @@
 // time loop, checkpoints, primitives) plus the small utility kernels and
 // k_ens, the batched-ensemble kernel.
 //
-// The DGSEM kernels themselves, k_visc and k_rhs, are templates in
+// The DGSEM kernels themselves are templates in
 // dg_device.h; their launch code (dg_launch.h) is instantiated per
 // (dimension, order) in inst.hip, and this unit calls those instances
 // through the PRANDTL_DISPATCH switch below.
@@ -433,7 +433,7 @@ int visc_only(prandtl_ctx *c, const double *y, double *grad, hipStream_t s)
     PRANDTL_DISPATCH(launch_visc, c, y, grad, s)
 }
 
-// k_rhs alone (mode 0, RHS into out); k_visc's outputs must be current
+// the RHS kernel alone (mode 0, RHS into out); the viscous kernel's outputs must be current
 int rhs_only(prandtl_ctx *c, const double *y, double *out, hipStream_t s)
 {
     PRANDTL_DISPATCH(launch_rhs, c, y, nullptr, out, 0, 0.0, 0.0, 0.0, s)
@@ -760,7 +760,6 @@ int create_impl(const prandtl_mesh_desc *mesh, const prandtl_quad_mesh *qm, cons
     c->geo.bcs = nullptr;
     for (int r = 0; r < dim && !umesh; r++)
         for (int side = 0; side < 2; side++) c->geo.bcmask |= mesh->bc[r][side] << (3 * (2 * r + side));
-    for (int i = 0; i < Np; i++) c->tab.fvs[i] = 1.0 / (J * w[i]);
     // subcell normals n_{i+1/2} = Ja + sum_{l<=i} w_l sum_q D_lq Ja (lines 1212-1233)
     for (int r = 0; r < dim; r++)
         for (int i = 1; i < Np; i++) {

@@ -27,7 +27,7 @@ struct prandtl_ctx {
     // kernel timing (prandtl_profile_begin/end): events bracketing every launch
     bool prof = false;
     std::vector<hipEvent_t> ev_pool;
-    std::vector<int> ev_kind;   // 0 = k_rhs, 1 = k_visc
+    std::vector<int> ev_kind;   // 0: RHS kernel, 1: viscous kernel
     size_t ev_used = 0;
     // SSP-RK3 step captured as a hipGraph (dt read from d_dt), replayed per step
     bool use_graph = true;
@@ -56,7 +56,7 @@ struct prandtl_ctx {
     double graph_dt = 0.0;        // value last copied to d_dt
     bool graph_dt_set = false;
     int rhs_algo = 0;             // PRANDTL_ALGO_TILE or _LINE (line_ok)
-    int rhs_shape = 0;            // k_rhs launch shape (only shapes rhs_shape_ok accepts are set)
+    int rhs_shape = 0;            // RHS launch shape (only shapes rhs_shape_ok accepts are set)
     int visc_shape = 0;           // k_visc / k_visc_l launch shape (visc_shape_ok)
     // device time loop (prandtl_run)
     LoopState *d_loop = nullptr;
@@ -316,11 +316,11 @@ int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
     ProfScope ps(c, s, 0);
     if constexpr (DIM == 1) {
-        using Cf = R1Cfg<NP, BLEND>;
-        const int nb = (c->NE + Cf::EPB - 1) / Cf::EPB;
-        if (c->geo.bcmask) hipLaunchKernelGGL((k_rhs<NP, BLEND, true>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-        else hipLaunchKernelGGL((k_rhs<NP, BLEND, false>), dim3(nb), dim3(Cf::BLOCK), 0, s, a);
-        return hip_check(c, hipGetLastError(), "k_rhs launch");
+        using Pc = PtCfg<DIM, NP>;
+        const dim3 nb((c->NE + Pc::EPB - 1) / Pc::EPB), bl(Pc::BLOCK);
+        if (c->geo.bcmask) hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, true, false>), nb, bl, 0, s, a);
+        else hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, false, false>), nb, bl, 0, s, a);
+        return hip_check(c, hipGetLastError(), "k_rhs_p launch");
     } else {
         if constexpr (gen_built(DIM, NP)) {
             if (c->gen) return launch_lines_sized<DIM, NP, BLEND, false, true>(c, a, s);

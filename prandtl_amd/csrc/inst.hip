@@ -1,4 +1,4 @@
-// One (dimension, order) pair of the k_visc / k_rhs launch templates and
+// One (dimension, order) pair of the viscous and RHS launch templates and
 // every kernel variant they launch, chosen by -DPRANDTL_INST_DIM and
 // -DPRANDTL_INST_NP: the Makefile builds one object per pair of
 // PRANDTL_ORDERS, in parallel.
