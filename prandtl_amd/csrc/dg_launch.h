@@ -131,12 +131,19 @@ template <int DIM, int NP, int FB, bool OPEN> void launch_visc_l(prandtl_ctx *c,
 // over more of them.  Euler right-hand sides, natural against this: 3-D N = 3
 // 512 elements 9.3 -> 8.0 us (2,197 elements 15.7 against 14.0, 4,096 18.6
 // against 18.7), N = 4 252 elements 10.8 -> 8.9, N = 2 125 elements 10.7 -> 8.5.
+// At N = 2, whose natural workgroup holds 9 elements, a single wave of 2 is
+// better up to 13,824 elements (4,096: RHS 11.5 -> 9.8, k_visc_l 9.5 -> 8.3;
+// 13,824: 23.0 -> 22.4, 18.5 both; 62,320: 87 against 89, 57 against 59).
 constexpr int lines_small_fb(int DIM, int NP) { return DIM != 3 || NP > 6 ? 0 : NP <= 4 ? 64 : 128; }
+template <int DIM, int NP> bool lines_small(const prandtl_ctx *c)
+{
+    return lines_small_fb(DIM, NP) > 0 && c->NE < (NP == 3 ? 1536 : 256) * LnCfg<DIM, NP>::EPB;
+}
 
 // Orders the general-geometry kernels are built for: 2-D N = 1..5, 3-D N = 2..4.
 constexpr bool gen_built(int DIM, int NP) { return DIM == 2 ? NP <= 6 : DIM == 3 && NP <= 5; }
 
-// The mixed form of the line algorithm on periodic 3-D boxes at N = 3 has no
+// The mixed form under PRANDTL_ALGO_LINE at N = 3 (periodic 3-D boxes) has no
 // choice of viscous launch shape.
 inline bool visc_shape_fixed(const prandtl_ctx *c)
 {
@@ -167,7 +174,7 @@ template <int DIM, int NP> int launch_visc_nd(prandtl_ctx *c, const double *y, d
     }
     if (!c->prm.quirks && !grad) {
         constexpr int SM = lines_small_fb(DIM, NP);
-        const bool small = SM > 0 && c->NE < 256 * LnCfg<DIM, NP>::EPB;
+        const bool small = lines_small<DIM, NP>(c);
         if (c->geo.bcmask) {
             if (small) launch_visc_l<DIM, NP, SM, true>(c, a, s);
             else launch_visc_l<DIM, NP, 0, true>(c, a, s);
@@ -306,7 +313,7 @@ int launch_lines_sized(prandtl_ctx *c, const KArgs &a, hipStream_t s)
     }
     constexpr int SM = lines_small_fb(DIM, NP);
     if constexpr (SM > 0) {
-        if (c->NE < 256 * LnCfg<DIM, NP>::EPB) return launch_lines<DIM, NP, BLEND, SM, OPEN, GEN>(c, a, s);
+        if (lines_small<DIM, NP>(c)) return launch_lines<DIM, NP, BLEND, SM, OPEN, GEN>(c, a, s);
     }
     return launch_lines<DIM, NP, BLEND, 0, OPEN, GEN>(c, a, s);
 }

@@ -38,8 +38,8 @@
 //  - The indicator's transforms run on the line threads: NP values in
 //    registers, NP^2 multiply-adds.
 //
-// Bound: FP64 issue and, next, HBM traffic; at three waves per SIMD (168
-// registers) neither is hidden completely.  3-D N = 7, 32^3 elements, blended
+// Bound: FP64 issue and, next, HBM traffic; at three or four waves per SIMD
+// neither is hidden completely.  3-D N = 7, 32^3 elements, blended
 // Navier-Stokes: 3,025 vector instructions per wave, 0.53 ms of issue and 3 GB,
 // 0.55 ms at the copy rate, in 0.95 ms (two waves per SIMD: 1.16 times
 // slower).  Against the kernel that took pairs as jobs, per right-hand side:
@@ -110,10 +110,7 @@ template <int DIM, int NP, int FB = 0> struct LnCfg {
     static constexpr int KP = NP == 6 ? K + K / NP : K;
     static constexpr int ES = NR * KP + (DIM == 3 && NP == 4 ? (NR * KP % 32 == 0 ? 16 : 0) : 0);
     static_assert(EPB >= 1, "a workgroup holds an element's lines");
-#ifndef PRANDTL_LINES_WAVES
-#define PRANDTL_LINES_WAVES 3
-#endif
-    static constexpr int WAVES = PRANDTL_LINES_WAVES;
+    static constexpr int WAVES = 3;
 };
 
 // Whether the pair and Vandermonde tables are read from LDS (broadcasts)
@@ -920,10 +917,20 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
     block_lam_max<BLOCK>(lam, lam_old, A.lam, S.Red, slot);
 }
 
+// Waves per SIMD to ask the register allocator for: 4 on 3-D boxes where 128
+// registers suffice but for a few spills (N = 3: 14; N = 2 blended: none), else
+// 3 (168).  45 x 43 x 41 N = 3 Navier-Stokes 228 -> 210 us per launch, mixed 251
+// -> 224, 40 x 41 x 39 blended Euler 209 -> 193, N = 2 108 -> 101; 16^3 the same
+// (its waves are 3 per SIMD).  2-D lines gain nothing from it (0.97 to 1.02).
+constexpr int lines_waves(int DIM, int NP, bool BLEND, bool QNS3, bool OPEN, bool GEN)
+{
+    return DIM == 3 && (NP == 4 || (NP == 3 && BLEND)) && !QNS3 && !OPEN && !GEN ? 4 : 3;
+}
+
 template <int DIM, int NP, bool BLEND, bool QNS3, typename VT, int FB, bool OPEN = false, bool GEN = false,
           bool AXI = false>
 __global__ void __launch_bounds__((LnCfg<DIM, NP, FB>::BLOCK))
-__attribute__((amdgpu_waves_per_eu((LnCfg<DIM, NP, FB>::WAVES)))) k_rhs_l(const KArgs A)
+__attribute__((amdgpu_waves_per_eu((lines_waves(DIM, NP, BLEND, QNS3, OPEN, GEN))))) k_rhs_l(const KArgs A)
 {
     __shared__ LineSmem<DIM, NP, BLEND, FB, GEN, AXI> S;
     line_body<DIM, NP, BLEND, QNS3, VT, FB, OPEN, GEN, AXI>(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.x, S);
