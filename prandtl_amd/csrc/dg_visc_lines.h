@@ -30,9 +30,9 @@
 //  D is applied in even-odd form (half the multiply-adds, and few enough
 //  entries for scalar registers), D^ as D and its boundary terms.
 //
-// Bound: latency at three to four waves per SIMD; at N = 7 1.37 GB of HBM
-// traffic (0.26 ms at the copy rate), 0.22 ms of vector issue and 0.16 ms of
-// LDS in 0.54 ms.  Against k_visc, which read a line's nodes once per node
+// Bound: latency at three to four waves per SIMD; at N = 7 1.8 GB of HBM
+// traffic (0.4 ms at the copy rate), 0.22 ms of vector issue and 0.16 ms of LDS
+// in 0.54 ms.  Against k_visc, which read a line's nodes once per node
 // (240 LDS reads per node at N = 7, 80 here) and took four logarithms per node
 // and face point, per launch: 3-D N = 3 16^3 17.2 -> 12.2 us, 45 x 43 x 41 208
 // -> 170, N = 7 32^3 686 -> 540; mixed N = 3 16^3 15.6 (on the FP32 matrix
