@@ -94,7 +94,7 @@ __device__ __forceinline__ NodeQ<DIM> node_quants(const double *s, const Phys &P
 //     series of 1/T to u^3 (the next terms are below 1e-17);
 //   u < 1/9 (y/x up to 2): T by a degree-10 polynomial, the Chebyshev
 //     interpolant of atanh(sqrt u)/sqrt u on [0, 1/9], relative error 2.4e-18;
-//   else (shocks, and every non-finite or negative value): (y-x)/log(y/x)
+//   else (shocks, values of two signs or not finite): (y-x)/log(y/x)
 //     with log(y/x) = k log 2 + log(y/(2^k x)), k the difference of the binary
 //     exponents, which brings the second logarithm into T's range: 45
 //     instructions against 130 of the library's logarithm and quotient.
@@ -122,13 +122,24 @@ __device__ __forceinline__ double atanh_ratio(double u)
     return fma(p, u, 1.0);
 }
 
-// T or log(y/x) of one mean in the third range's form: k = 0 (a ratio inside
-// (1/2, 2)) gives T(u) as the second range does; otherwise log(y/x), NaN for
-// values of different sign, as the logarithm of their quotient is.  log 2 in
-// two parts, the first with trailing zeros, so that k times it is exact.
+// Whether the second range's formulas hold: values of one sign within a ratio
+// of 2 of each other, |y - x| < min(|x|, |y|).  The difference is exact where it
+// decides, so a pair between two values that pass the test passes it too.  (A
+// negative density or pressure, in a state that has lost its physics, still has
+// a mean while its neighbours are negative as well.)
+__device__ __forceinline__ bool lm_inside(double x, double y)
+{
+    return fabs(y - x) < fmin(fabs(x), fabs(y));
+}
+
+// T or log(y/x) of one mean in the third range's form: k = 0 (lm_inside) gives
+// T(u) as the second range does; otherwise log(y/x), NaN for values of different
+// sign, as the logarithm of their quotient is.  log 2 in two parts: the double
+// with its last 21 bits cut off, so that k times it is exact, and the double
+// nearest the rest.
 __device__ __forceinline__ bool log_parts(double x, double y, double &TL)
 {
-    const bool in = (y < x + x) & (x < y + y);
+    const bool in = lm_inside(x, y);
     const int k = in ? 0 : __builtin_amdgcn_frexp_exp(y) - __builtin_amdgcn_frexp_exp(x);
     const double xk = ldexp(x, k);
     const double f = (y - xk) * rcp_nr(xk + y);
@@ -143,7 +154,7 @@ __device__ __forceinline__ bool log_parts(double x, double y, double &TL)
 // ratio of a whole line's values; LM_MID the second (and valid in the first);
 // LM_ANY every value, by the second range's formulas where they hold.  Where
 // both hold MID and ANY agree bitwise, so a wave may take ANY for all its
-// lanes as soon as one of them needs it (lm_any below) without a lane's
+// lanes as soon as one of them needs it (ec_flux below) without a lane's
 // result depending on the others.
 enum { LM_SHORT = 0, LM_MID = 1, LM_ANY = 2, LM_PAIR = 3 };
 
@@ -175,9 +186,6 @@ __device__ __forceinline__ void log_means(double ra, double rb, double ba, doubl
         }
     }
 }
-
-// Whether the second range's formulas do not hold for the pair.
-__device__ __forceinline__ bool lm_outside(double x, double y) { return !((y < x + x) & (x < y + y)); }
 
 // Chandrashekar two-point flux for the normal (or mean metric) vector n.
 // DISS = false: ComputeVolumeFlux (ChandrashekarFlux.cpp:11-83).  DISS =
@@ -242,7 +250,7 @@ __device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<
 {
     if (TRY_SHORT && ((fabs(b.rho - a.rho) < 0.01 * (a.rho + b.rho)) & (fabs(b.beta - a.beta) < 0.01 * (a.beta + b.beta))))
         ec_flux_r<DIM, DISS, LM_SHORT>(n, nd, a, b, P, quirk3d, F);
-    else if (__any(lm_outside(a.rho, b.rho) | lm_outside(a.beta, b.beta)))
+    else if (!__all(lm_inside(a.rho, b.rho) & lm_inside(a.beta, b.beta)))
         ec_flux_r<DIM, DISS, LM_ANY>(n, nd, a, b, P, quirk3d, F);
     else ec_flux_r<DIM, DISS, LM_MID>(n, nd, a, b, P, quirk3d, F);
 }
