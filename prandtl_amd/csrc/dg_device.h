@@ -68,6 +68,7 @@ struct Geo {
     double inv_n0, inv_n01;   // 1 / n[0], 1 / (n[0] n[1]): box element index arithmetic
     double invJ;     // 1/J
     double aface;    // 1/(w_0 J)
+    double nsc, insc;   // meshes: the power of two that brings the largest normal near 1, and its inverse
     int bcmask;      // boundary type (BC_*) of side (r, s) in bits 3(2r+s)..+2; 0: periodic box
     const double *bcs;    // device outer states of inflow / specified-state boundaries, 5 per
                           // box side [3][2] (Cartesian) or per attribute (unstructured meshes)

@@ -728,6 +728,12 @@ int create_impl(const prandtl_mesh_desc *mesh, const prandtl_quad_mesh *qm, cons
         c->gen = true;
         c->hmin = qg.hmin;
     }
+    double nmax = 0.0;
+    for (double v : qg.fnor) nmax = std::max(nmax, std::fabs(v));
+    int nexp = 0;
+    (void)std::frexp(nmax, &nexp);
+    c->geo.nsc = std::ldexp(1.0, -nexp);
+    c->geo.insc = std::ldexp(1.0, nexp);
     // Cartesian geometry: J = det diag(h), adj = diag of cofactors
     double h[3] = {1, 1, 1};
     for (int r = 0; r < dim; r++) {

@@ -566,12 +566,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
 #pragma unroll
             for (int d = 0; d < DIM; d++) { q1.v[d] = own ? qo.v[d] : qn.v[d]; q2.v[d] = own ? qn.v[d] : qo.v[d]; }
             if constexpr (GEN) {
-                double nn[DIM], n2 = nv[side][0] * nv[side][0];
-#pragma unroll
-                for (int d = 0; d < DIM; d++) nn[d] = nv[side][d];
-#pragma unroll
-                for (int d = 1; d < DIM; d++) n2 = fma(nn[d], nn[d], n2);
-                ec_flux<DIM, true, DIM == 3>(nn, sqrt(n2), q1, q2, P, quirk3d, F);
+                ec_flux<DIM, true, DIM == 3>(nv[side], normal_length<DIM>(nv[side], A.geo.nsc, A.geo.insc), q1, q2, P, quirk3d, F);
             } else {
                 if (A.ec) ec_flux<DIM, false>(nvec, nr, q1, q2, P, false, F);
                 else ec_flux<DIM, true, DIM == 3>(nvec, nr, q1, q2, P, quirk3d, F);
@@ -813,10 +808,9 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                     double ns[DIM], nd;
                     if constexpr (GEN) {
                         const double *sn = A.geo.subn + ((((size_t)e * DIM + r) * NFP + l) * (NP - 1) + i) * DIM;
-                        nd = 0.0;
 #pragma unroll
-                        for (int d = 0; d < DIM; d++) { ns[d] = sn[d]; nd = fma(ns[d], ns[d], nd); }
-                        nd = sqrt(nd);
+                        for (int d = 0; d < DIM; d++) ns[d] = sn[d];
+                        nd = normal_length<DIM>(ns, A.geo.nsc, A.geo.insc);
                         if constexpr (AXI) {
                             // flux_num *= mid_r (DGSEMIntegrator.cpp:1030-1032, 1110-1112)
                             const double rh = 0.5 * (S.R[el][ls[i]] + S.R[el][ls[i + 1]]);

@@ -298,10 +298,21 @@ __device__ __forceinline__ double norml2_3(const double *n)
     return scale * sqrt(sum);
 }
 
-template <int DIM> __device__ __forceinline__ double norml2_v(const double *n)
+// |n| of a mesh's face or subcell normal: the squares of the components times sc,
+// a power of two that brings the mesh's largest normal near 1 (isc = 1/sc), so
+// that they neither under- nor overflow (normals of 3-D meshes are squares of
+// lengths).  The scaling is exact: the result is that of the plain sum where
+// that is in range.
+template <int DIM>
+__device__ __forceinline__ double normal_length(const double *n, double sc, double isc)
 {
-    if constexpr (DIM == 2) return norml2_2(n);
-    else return norml2_3(n);
+    double s = 0.0;
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        const double x = n[d] * sc;
+        s = (d == 0) ? x * x : fma(x, x, s);
+    }
+    return sqrt(s) * isc;
 }
 
 // Boundary types (PRANDTL_BC_*)

@@ -280,12 +280,7 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
 #pragma unroll
             for (int d = 0; d < DIM; d++) { q1.v[d] = own ? qo.v[d] : qn.v[d]; q2.v[d] = own ? qn.v[d] : qo.v[d]; }
             if constexpr (GEN) {
-                double nn[DIM], nsq = nv[0] * nv[0];
-#pragma unroll
-                for (int d = 0; d < DIM; d++) nn[d] = nv[d];
-#pragma unroll
-                for (int d = 1; d < DIM; d++) nsq = fma(nn[d], nn[d], nsq);
-                ec_flux<DIM, true, DIM == 3>(nn, sqrt(nsq), q1, q2, P, quirk3d, F);
+                ec_flux<DIM, true, DIM == 3>(nv, normal_length<DIM>(nv, A.geo.nsc, A.geo.insc), q1, q2, P, quirk3d, F);
             } else {
                 if (A.ec) ec_flux<DIM, false>(nvec, nr, q1, q2, P, false, F);
                 else ec_flux<DIM, true, DIM == 3>(nvec, nr, q1, q2, P, quirk3d, F);
@@ -436,10 +431,9 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
                     double ns[DIM], nd;
                     if constexpr (GEN) {
                         const double *sv = A.geo.subn + ((((size_t)e * DIM + r) * NFP + l) * (NP - 1) + i) * DIM;
-                        nd = 0.0;
 #pragma unroll
-                        for (int d = 0; d < DIM; d++) { ns[d] = sv[d]; nd = fma(ns[d], ns[d], nd); }
-                        nd = sqrt(nd);
+                        for (int d = 0; d < DIM; d++) ns[d] = sv[d];
+                        nd = normal_length<DIM>(ns, A.geo.nsc, A.geo.insc);
                     } else {
                         nd = A.tab.subn[0][0];
 #pragma unroll

@@ -5,7 +5,9 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
-from prandtl_amd import DGSEMOperator
+import quad_meshes as Q
+from prandtl_amd import DGSEMOperator, cases
+from prandtl_amd.operator import HexMesh
 
 pytestmark = pytest.mark.gpu
 
@@ -52,4 +54,23 @@ def test_negative_values(cuda, dim, order, n, rho0, p0, ec, equal):
     assert np.isfinite(out).all()
     r = rel_max(out, ref)
     print("%dD N=%d %g %g ec=%d equal=%d: %.2e" % (dim, order, rho0, p0, ec, equal, r), flush=True)
+    assert r <= TOL
+
+
+@pytest.mark.parametrize("size", [1e-80, 1.0, 1e80])
+@pytest.mark.parametrize("order,n", [(2, 3), (3, 3), (3, 11), (4, 3)])
+def test_mesh_size(cuda, order, n, size):
+    """Hexahedra whose normals' squares are out of range: the normals are squares
+    of lengths, the right-hand side (of an Euler state) is a rate per length."""
+    d = Q.hex_grid(n, 3, n, (0.0,) * 3, (size, 0.8 * size, 0.6 * size), periodic=(False, True, True), perturb=0.2, seed=1)
+    d.update(attr_bc=["slip", "symmetry"], attr_state=[(0.0,) * 5] * 2)
+    mesh = HexMesh(d["vert"], d["elem"], d["bdr"], d["bdr_attr"], d["elem_coords"])
+    kw = dict(blending=True, quirks=False)
+    op = DGSEMOperator.hex(mesh, order, bc={1: "slip", 2: "symmetry"}, **kw)
+    orc = O.Oracle.hex(d, order, threads=16, **kw)
+    u = cases.random_smooth_state(orc.coords() / size, 3, 3, L=[1.0, 0.8, 0.6])
+    out, ref = mult(op, u, cuda), orc.Mult(u)
+    assert np.isfinite(ref).all()
+    r = rel_max(out, ref)
+    print("N=%d %d size %g: %.2e" % (order, n, size, r), flush=True)
     assert r <= TOL
