@@ -337,16 +337,20 @@ __device__ __forceinline__ double slip_wall_flux(int r, double ns, const double 
     // 1-D: state2(1) * nor(0) (SlipWallBdrFaceIntegrator.cpp:22-30)
     if constexpr (DIM == 1) m[0] = s[1] * ns;
     if constexpr (DIM == 2) {
-        m[0] = (r == 0 ? s[1] : s[2]) * u;
-        m[1] = r == 0 ? s[2] * u : -(s[1] * u);
+        const double s1 = s[1], s2 = s[2];
+        m[0] = (r == 0 ? s1 : s2) * u;
+        m[1] = r == 0 ? s2 * u : -(s1 * u);
     }
     if constexpr (DIM == 3) {
         // selects, not branches: r differs between the lanes of a wave, and
         // the compiler (ROCm 7.2), sinking the -s[1] that the branches for
-        // r = 1 and r = 2 share, left m[1] unset in the lanes with r = 2
-        m[0] = (r == 0 ? s[1] : r == 1 ? s[2] : s[3]) * u;
-        m[1] = r == 0 ? s[2] : -s[1];
-        m[2] = r == 2 ? -(s[2] * u) : s[3] * u;
+        // r = 1 and r = 2 share, left m[1] unset in the lanes with r = 2.
+        // Between values already loaded: a choice of elements of s would put
+        // the caller's state into scratch memory
+        const double s1 = s[1], s2 = s[2], s3 = s[3];
+        m[0] = (r == 0 ? s1 : r == 1 ? s2 : s3) * u;
+        m[1] = r == 0 ? s2 : -s1;
+        m[2] = r == 2 ? -(s2 * u) : s3 * u;
     }
     // Conserv2Prim (BasicOperations.cpp:172-186): velocities by division,
     // the pressure's by the reciprocal (ComputePressure, lines 31-37)
