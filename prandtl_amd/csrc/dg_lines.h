@@ -784,16 +784,15 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                 rlo = fmin(rlo, a); rhi = fmax(rhi, a);
                 blo = fmin(blo, b); bhi = fmax(bhi, b);
             }
-            // a pair of a line whose extremes have one sign has at most their
-            // ratio; extremes of two signs fail both tests.  (fmin and fmax drop
-            // a NaN, which then reaches its pairs' fluxes in any range.)  SHORT,
-            // where a line's values are positive and differ by at most 2%, in
-            // 3-D only: in 2-D more waves hold lines of both kinds, and would
-            // run two loops
+            // a pair's ratio is at most that of the line's extremes (positive
+            // values; others fail both tests, but for a NaN, which fmin and
+            // fmax drop and which makes its pairs' fluxes NaN in any range).
+            // SHORT, where a line's values differ by at most 2%, in 3-D only: in
+            // 2-D more waves hold lines of both kinds, and would run two loops
             const double dr = rhi - rlo, rs = rhi + rlo, db = bhi - blo, bs = bhi + blo;
             if (DIM == 3 && ((dr < 0.01 * rs) & (db < 0.01 * bs))) pairs(std::integral_constant<int, LM_SHORT>{});
             else if constexpr (NP >= 7) pairs(std::integral_constant<int, LM_PAIR>{});   // (registers)
-            else if (!__all(lm_inside(rlo, rhi) & lm_inside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
+            else if (__any(lm_outside(rlo, rhi) | lm_outside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
             else pairs(std::integral_constant<int, LM_MID>{});
         }
 

@@ -122,24 +122,17 @@ __device__ __forceinline__ double atanh_ratio(double u)
     return fma(p, u, 1.0);
 }
 
-// Whether the second range's formulas hold: values of one sign within a ratio
-// of 2 of each other, |y - x| < min(|x|, |y|).  The difference is exact where it
-// decides, so a pair between two values that pass the test passes it too.  (A
-// negative density or pressure, in a state that has lost its physics, still has
-// a mean while its neighbours are negative as well.)
-__device__ __forceinline__ bool lm_inside(double x, double y)
-{
-    return fabs(y - x) < fmin(fabs(x), fabs(y));
-}
-
-// T or log(y/x) of one mean in the third range's form: k = 0 (lm_inside) gives
-// T(u) as the second range does; otherwise log(y/x), NaN for values of different
-// sign, as the logarithm of their quotient is.  log 2 in two parts: the double
-// with its last 21 bits cut off, so that k times it is exact, and the double
-// nearest the rest.
+// T or log(y/x) of one mean in the third range's form: T(u), as the second range
+// has it, for values of one sign within a ratio of 2, |y - x| < min(|x|, |y|)
+// (exact where it decides; negative values, of a state that has lost its
+// physics, have a mean while both are negative); otherwise log(y/x), NaN for
+// values of different sign, as the logarithm of their quotient is.  log 2 in two
+// parts: the double with its last 21 bits cut off, so that k times it is exact,
+// and the double nearest the rest.
 __device__ __forceinline__ bool log_parts(double x, double y, double &TL)
 {
-    const bool in = lm_inside(x, y);
+    const double d = fabs(y - x);
+    const bool in = (d < fabs(x)) & (d < fabs(y));
     const int k = in ? 0 : __builtin_amdgcn_frexp_exp(y) - __builtin_amdgcn_frexp_exp(x);
     const double xk = ldexp(x, k);
     const double f = (y - xk) * rcp_nr(xk + y);
@@ -186,6 +179,10 @@ __device__ __forceinline__ void log_means(double ra, double rb, double ba, doubl
         }
     }
 }
+
+// Whether the second range's formulas do not hold for the pair, or its values
+// are not positive.
+__device__ __forceinline__ bool lm_outside(double x, double y) { return !((y < x + x) & (x < y + y)); }
 
 // Chandrashekar two-point flux for the normal (or mean metric) vector n.
 // DISS = false: ComputeVolumeFlux (ChandrashekarFlux.cpp:11-83).  DISS =
@@ -250,7 +247,7 @@ __device__ __forceinline__ void ec_flux(const double *n, double nd, const NodeQ<
 {
     if (TRY_SHORT && ((fabs(b.rho - a.rho) < 0.01 * (a.rho + b.rho)) & (fabs(b.beta - a.beta) < 0.01 * (a.beta + b.beta))))
         ec_flux_r<DIM, DISS, LM_SHORT>(n, nd, a, b, P, quirk3d, F);
-    else if (!__all(lm_inside(a.rho, b.rho) & lm_inside(a.beta, b.beta)))
+    else if (__any(lm_outside(a.rho, b.rho) | lm_outside(a.beta, b.beta)))
         ec_flux_r<DIM, DISS, LM_ANY>(n, nd, a, b, P, quirk3d, F);
     else ec_flux_r<DIM, DISS, LM_MID>(n, nd, a, b, P, quirk3d, F);
 }

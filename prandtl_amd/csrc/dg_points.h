@@ -417,7 +417,7 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
         }
         const double dr = rhi - rlo, rs = rhi + rlo, db = bhi - blo, bs = bhi + blo;
         if (DIM == 3 && ((dr < 0.01 * rs) & (db < 0.01 * bs))) pairs(std::integral_constant<int, LM_SHORT>{});
-        else if (!__all(lm_inside(rlo, rhi) & lm_inside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
+        else if (__any(lm_outside(rlo, rhi) | lm_outside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
         else pairs(std::integral_constant<int, LM_MID>{});
 
         if constexpr (BLEND) {
