@@ -368,26 +368,48 @@ __device__ __forceinline__ double ax_clamp(double x, double m)
     return x > 0.0 ? m : (x < 0.0 ? -m : 0.0);
 }
 
-__device__ __forceinline__ void axis_node(const double *rU, const Geo &g, int K, size_t NK, size_t q, double U[4])
+// What a node's recovery loads in any case.  Apart from the rest, so that a
+// thread with several nodes has all of these loads in flight at once.
+struct AxNode {
+    int code;
+    double r, u[4];
+};
+
+__device__ __forceinline__ AxNode axis_load(const double *rU, const Geo &g, size_t NK, size_t q)
 {
-    const int code = g.axm[q];
-    if (code < 0) {
-        const double r = g.rnode[q];
+    AxNode n;
+    n.code = g.axm[q];
+    n.r = g.rnode[q];
 #pragma unroll
-        for (int v = 0; v < 4; v++) U[v] = rU[v * NK + q] / r;
+    for (int v = 0; v < 4; v++) n.u[v] = rU[v * NK + q];
+    return n;
+}
+
+__device__ __forceinline__ void axis_state(const double *rU, const Geo &g, int K, size_t NK, size_t q, const AxNode &n,
+                                           double U[4])
+{
+    if (n.code < 0) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) U[v] = n.u[v] / n.r;
         return;
     }
-    const int d = code >> 1;
+    const int d = n.code >> 1;
     const size_t eb = q - q % (size_t)K;
     const int j1 = g.axj[3 * d], j2 = g.axj[3 * d + 1], jn = g.axj[3 * d + 2];
     const double r1 = g.axr[3 * d], r2 = g.axr[3 * d + 1], rn = g.axr[3 * d + 2];
+    double f1s[4], f2s[4], fns[4];   // (loaded together; no node: node 0, unused)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        f1s[v] = rU[v * NK + eb + (j1 < 0 ? 0 : j1)];
+        f2s[v] = rU[v * NK + eb + (j2 < 0 ? 0 : j2)];
+        fns[v] = rU[v * NK + eb + jn];
+    }
     auto fit = [&](int comp) -> double {
         if (j1 < 0) return 0.0;
-        const double f1 = rU[comp * NK + eb + j1];
+        const double f1 = f1s[comp], f2 = f2s[comp];
         const double fref = fabs(f1);
         const double cap = (fref < 1e-12) ? INFINITY : 10.0 * fref / fmax(r1, 1e-14);
         if (j2 >= 0) {
-            const double f2 = rU[comp * NK + eb + j2];
             const double m = (r1 * f1 + r2 * f2) / fmax(r1 * r1 + r2 * r2, 1e-14);
             return ax_clamp(ax_minmod(m, ax_minmod(1.5 * (f1 / r1), 1.5 * (f2 / r2))), cap);
         }
@@ -396,7 +418,7 @@ __device__ __forceinline__ void axis_node(const double *rU, const Geo &g, int K,
     const double rho = fit(0), mz = fit(1), E = fit(3);
     if (!isfinite(rho) || rho < g.axis_floor || !isfinite(E)) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) U[v] = rU[v * NK + eb + jn] / rn;
+        for (int v = 0; v < 4; v++) U[v] = fns[v] / rn;
         U[2] = 0.0;
     } else {
         U[0] = rho;

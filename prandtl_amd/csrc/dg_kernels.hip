@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(256) k_axis(const double *rU, double *U, Geo g
     const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= NK) return;
     double u[4];
-    axis_node(rU, g, K, NK, q, u);
+    axis_state(rU, g, K, NK, q, axis_load(rU, g, NK, q), u);
 #pragma unroll
     for (int v = 0; v < 4; v++) U[v * NK + q] = u[v];
 }

@@ -308,12 +308,14 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
         }
     }
     double ysp[NPASS][NV];
+    AxNode xn[AXI ? NPASS : 1], xt[AXI ? 2 : 1];
+    size_t gt[2] = {0, 0};
 #pragma unroll
     for (int p = 0; p < NPASS; p++) {
         const int i = t + p * BLOCK;
         const size_t gi = (i < nact) ? (size_t)ebase * K + i : 0;
         if constexpr (AXI) {
-            axis_node(A.y, A.geo, K, NK, gi, ysp[p]);
+            xn[p] = axis_load(A.y, A.geo, NK, gi);
         } else {
 #pragma unroll
             for (int v = 0; v < NV; v++) {
@@ -346,7 +348,8 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
             g = lact ? (size_t)en * K + nn : 0;
         }
         if constexpr (AXI) {
-            axis_node(A.y, A.geo, K, NK, g, pt[side]);
+            xt[side] = axis_load(A.y, A.geo, NK, g);
+            gt[side] = g;
         } else {
 #pragma unroll
             for (int v = 0; v < NV; v++) {
@@ -421,6 +424,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
         if (i >= nact) continue;
         const int e2 = EPB == 1 ? 0 : i / K, n = i - e2 * K;
         const int s = lines_node_slot<DIM, NP>(n);
+        if constexpr (AXI) axis_state(A.y, A.geo, K, NK, (size_t)ebase * K + i, xn[p], ysp[p]);
         const NodeQ<DIM> q = node_quants<DIM>(ysp[p], P);
         sQ(e2, 0, s) = q.rho;
 #pragma unroll
@@ -479,6 +483,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
         for (int side = 0; side < 2; side++) {
             double *pn = pt[side];
             const int mo = side ? NP - 1 : 0;
+            if constexpr (AXI) axis_state(A.y, A.geo, K, NK, gt[side], xt[side], pn);
             double F[NV];
             if ((OPEN || GEN) && bt[side] != BC_PERIODIC) {
                 // boundary point: F_b for the outward normal at the interior
