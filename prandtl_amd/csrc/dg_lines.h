@@ -765,7 +765,8 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                             for (int d = 0; d < DIM; d++) n1[d] = d == 1 ? om * A.geo.nrm[1] : 0.0;
                         }
                         double g[NV];
-                        ec_flux<DIM, false>(n1, 0.0, qa, qe, P, false, g);
+                        if constexpr (RANGE == LM_PAIR) ec_flux<DIM, false>(n1, 0.0, qa, qe, P, false, g);
+                        else ec_flux_r<DIM, false, RANGE>(n1, 0.0, qa, qe, P, false, g);
 #pragma unroll
                         for (int b = a + 1; b < NP; b++)
 #pragma unroll
@@ -777,9 +778,9 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                 }
             }
         };
-        if constexpr (QNS3) {
-            // the range pair by pair: the second flux per node leaves no
-            // registers for separate loops
+        if constexpr (QNS3 && GEN) {
+            // the range pair by pair: the second flux per node and its metrics
+            // leave no registers for separate loops
             pairs(std::integral_constant<int, LM_PAIR>{});
         } else {
             double rlo = sQ(el, 0, ls[0]), rhi = rlo, blo = sQ(el, NV - 1, ls[0]), bhi = blo;
@@ -789,13 +790,26 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                 rlo = fmin(rlo, a); rhi = fmax(rhi, a);
                 blo = fmin(blo, b); bhi = fmax(bhi, b);
             }
+            if constexpr (QNS3) {
+                // and the zeta partners' second nodes
+                if (r == 2 && lb < NP - 1)
+#pragma unroll
+                    for (int m = 0; m < NP - 1; m++) {
+                        const int se = lines_slot<DIM, NP>(la, NP - 1, m);
+                        const double a = sQ(el, 0, se), b = sQ(el, NV - 1, se);
+                        rlo = fmin(rlo, a); rhi = fmax(rhi, a);
+                        blo = fmin(blo, b); bhi = fmax(bhi, b);
+                    }
+            }
             // a pair's ratio is at most that of the line's extremes (positive
             // values; others fail both tests, but for a NaN, which fmin and
             // fmax drop and which makes its pairs' fluxes NaN in any range).
             // SHORT, where a line's values differ by at most 2%, in 3-D only: in
-            // 2-D more waves hold lines of both kinds, and would run two loops
+            // 2-D more waves hold lines of both kinds, and would run two loops,
+            // as would the faithful NS-3D form on coarse meshes, whose loops are
+            // long (N = 6, 210 elements 32 us without, 40 with)
             const double dr = rhi - rlo, rs = rhi + rlo, db = bhi - blo, bs = bhi + blo;
-            if (DIM == 3 && ((dr < 0.01 * rs) & (db < 0.01 * bs))) pairs(std::integral_constant<int, LM_SHORT>{});
+            if (DIM == 3 && !QNS3 && ((dr < 0.01 * rs) & (db < 0.01 * bs))) pairs(std::integral_constant<int, LM_SHORT>{});
             else if constexpr (NP >= 7) pairs(std::integral_constant<int, LM_PAIR>{});   // (registers)
             else if (__any(lm_outside(rlo, rhi) | lm_outside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
             else pairs(std::integral_constant<int, LM_MID>{});
