@@ -134,9 +134,13 @@ template <int DIM, int NP, int FB, bool OPEN> void launch_visc_l(prandtl_ctx *c,
 // At N = 2, whose natural workgroup holds 9 elements, a single wave of 2 is
 // better up to 13,824 elements (4,096: RHS 11.5 -> 9.8, k_visc_l 9.5 -> 8.3;
 // 13,824: 23.0 -> 22.4, 18.5 both; 62,320: 87 against 89, 57 against 59).
+// Not the faithful NS-3D form at N = 4, whose small workgroup fills 75 of 128
+// threads: 720 elements 27.7 -> 25.6, walls 32.8 -> 30.1, hexahedra 35.2 -> 33.6.
+inline bool qns3(const prandtl_ctx *c) { return c->dim == 3 && c->prm.parabolic && c->prm.quirks; }
 constexpr int lines_small_fb(int DIM, int NP) { return DIM != 3 || NP > 6 ? 0 : NP <= 4 ? 64 : 128; }
 template <int DIM, int NP> bool lines_small(const prandtl_ctx *c)
 {
+    if (NP == 5 && qns3(c)) return false;
     return lines_small_fb(DIM, NP) > 0 && c->NE < (NP == 3 ? 1536 : 256) * LnCfg<DIM, NP>::EPB;
 }
 
@@ -247,33 +251,42 @@ inline bool line_default(const prandtl_ctx *c)
     return line_ok(c) && (c->Np <= 4 || c->prm.blending);
 }
 
-// One instance of k_rhs_l: the faithful NS-3D form, the mixed form or plain FP64.
+// The form of the right-hand side a context's equations take: calls f with
+// (QNS3, element type of the viscous terms, AXI) as constants: the faithful NS-3D
+// form, the mixed form, an axisymmetric mesh, or plain FP64.
+template <int DIM, bool GEN, typename Fn> void rhs_form(const prandtl_ctx *c, Fn f)
+{
+    using std::false_type;
+    using std::true_type;
+    if constexpr (DIM == 2 && GEN)
+        if (c->axi) return f(false_type{}, 0.0, true_type{});
+    if constexpr (DIM == 3)
+        if (qns3(c)) return f(true_type{}, 0.0, false_type{});
+    if constexpr (DIM > 1)
+        if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED) return f(false_type{}, 0.0f, false_type{});
+    f(false_type{}, 0.0, false_type{});
+}
+
 template <int DIM, int NP, bool BLEND, int FB, bool OPEN, bool GEN>
 int launch_lines(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
     using Lc = LnCfg<DIM, NP, FB>;
-    const dim3 nb((c->NE + Lc::EPB - 1) / Lc::EPB), bl(Lc::BLOCK);
-    if constexpr (DIM == 2 && GEN) {
-        if (c->axi) {
-            // the axisymmetric RHS (Euler), recovering U from r U as it loads
-            hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, double, FB, OPEN, GEN, true>), nb, bl, 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_rhs_l launch");
-        }
-    }
-    if constexpr (DIM == 3) {
-        if (c->prm.parabolic && c->prm.quirks) {
-            hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, true, double, FB, OPEN, GEN>), nb, bl, 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_rhs_l launch");
-        }
-    }
-    if constexpr (DIM > 1) {
-        if (c->prm.parabolic && c->prm.precision == PRANDTL_MIXED) {
-            hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, float, FB, OPEN, GEN>), nb, bl, 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_rhs_l launch");
-        }
-    }
-    hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, false, double, FB, OPEN, GEN>), nb, bl, 0, s, a);
+    rhs_form<DIM, GEN>(c, [&](auto q, auto vt, auto axi) {
+        hipLaunchKernelGGL((k_rhs_l<DIM, NP, BLEND, decltype(q)::value, decltype(vt), FB, OPEN, GEN, decltype(axi)::value>),
+                           dim3((c->NE + Lc::EPB - 1) / Lc::EPB), dim3(Lc::BLOCK), 0, s, a);
+    });
     return hip_check(c, hipGetLastError(), "k_rhs_l launch");
+}
+
+template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN>
+int launch_points(prandtl_ctx *c, const KArgs &a, hipStream_t s)
+{
+    using Pc = PtCfg<DIM, NP>;
+    rhs_form<DIM, GEN>(c, [&](auto q, auto vt, auto axi) {
+        hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, decltype(q)::value, decltype(vt), OPEN, GEN, decltype(axi)::value>),
+                           dim3((c->NE + Pc::EPB - 1) / Pc::EPB), dim3(Pc::BLOCK), 0, s, a);
+    });
+    return hip_check(c, hipGetLastError(), "k_rhs_p launch");
 }
 
 // Whether a mesh takes k_rhs_p instead of k_rhs_l: by the waves its node
@@ -287,29 +300,41 @@ int launch_lines(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 //   3-D N = 2 blended 336 11.1 / 10.3, 1,716 11.6 / 13.2 (without blending no gain);
 //   N = 3 120 hexahedra 10.4 / 8.2, 720 10.0 / 10.5; N = 4 210 10.6 / 8.6, 336
 //   hexahedra 12.8 / 16.1; N = 5 210 14.0 / 11.2, 336 14.4 / 18.1.
-template <int DIM, int NP, bool BLEND, bool GEN> constexpr int points_waves()
+// Where the line's chain is longer still, later:
+//   axisymmetric (a line thread recovers up to five nodes' states): N = 1 14,520
+//   quadrilaterals 13.7 / 10.7, N = 2 10,100 16.6 / 14.9, 14,520 17.1 / 17.3, N = 3
+//   6,480 16.9 / 15.4, 10,100 17.9 / 18.1, N = 4 4,160 18.9 / 18.0, 6,480 21.0 /
+//   22.5, N = 5 3,192 20.7 / 19.3, 4,160 21.4 / 22.6;
+//   2-D walls: N = 4 3,192 12.7 / 12.2, 4,160 12.8 / 14.1, N = 5 2,352 14.6 / 13.0,
+//   3,192 14.8 / 15.6;
+//   faithful NS-3D: N = 3 walls 504 23.2 / 21.1, 720 23.2 / 22.6, 990 23.3 / 24.0, N =
+//   4 336 25.2 / 21.6, 504 25.6 / 22.1, 720 27.7 / 27.8, walls 504 30.5 / 25.1, 720 32.8
+//   / 31.6, but hexahedra 336 31.1 / 33.0.
+template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN> int points_waves(const prandtl_ctx *c)
 {
-    if (DIM == 2) return NP == 2 ? 768 : NP == 3 ? 1792 : NP == 4 ? 2048 : NP == 5 && !BLEND && !GEN ? 1792 : 3072;
+    if constexpr (DIM == 2) {
+        if (GEN && c->axi) return NP == 2 ? 1920 : NP <= 4 ? 3584 : 4608;
+        if (OPEN && !BLEND && NP >= 5) return 3328;
+        return NP == 2 ? 768 : NP == 3 ? 1792 : NP == 4 ? 2048 : NP == 5 && !BLEND && !GEN ? 1792 : 3072;
+    }
+    if constexpr (!BLEND) {
+        if (qns3(c) && NP == 4 && (OPEN || GEN)) return 2304;
+        if (qns3(c) && NP == 5 && !GEN) return 3328;
+    }
     return NP == 3 ? (BLEND ? 512 : 0) : NP == 4 ? 1024 : NP == 5 ? 1536 : 2560;
 }
 
-template <int DIM, int NP, bool BLEND, bool GEN> bool points_ok(const prandtl_ctx *c)
+template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN> bool points_ok(const prandtl_ctx *c)
 {
     using Pc = PtCfg<DIM, NP>;
-    if (c->axi || (c->prm.parabolic && (c->prm.quirks || c->prm.precision == PRANDTL_MIXED))) return false;
-    return (long long)(c->NE + Pc::EPB - 1) / Pc::EPB * (Pc::BLOCK / 64) <= points_waves<DIM, NP, BLEND, GEN>();
+    return (long long)(c->NE + Pc::EPB - 1) / Pc::EPB * (Pc::BLOCK / 64) <= points_waves<DIM, NP, BLEND, OPEN, GEN>(c);
 }
 
 template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN>
 int launch_lines_sized(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
     if constexpr (points_built(DIM, NP)) {
-        if (points_ok<DIM, NP, BLEND, GEN>(c)) {
-            using Pc = PtCfg<DIM, NP>;
-            hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, OPEN, GEN>), dim3((c->NE + Pc::EPB - 1) / Pc::EPB),
-                               dim3(Pc::BLOCK), 0, s, a);
-            return hip_check(c, hipGetLastError(), "k_rhs_p launch");
-        }
+        if (points_ok<DIM, NP, BLEND, OPEN, GEN>(c)) return launch_points<DIM, NP, BLEND, OPEN, GEN>(c, a, s);
     }
     constexpr int SM = lines_small_fb(DIM, NP);
     if constexpr (SM > 0) {
@@ -323,11 +348,8 @@ int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
 {
     ProfScope ps(c, s, 0);
     if constexpr (DIM == 1) {
-        using Pc = PtCfg<DIM, NP>;
-        const dim3 nb((c->NE + Pc::EPB - 1) / Pc::EPB), bl(Pc::BLOCK);
-        if (c->geo.bcmask) hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, true, false>), nb, bl, 0, s, a);
-        else hipLaunchKernelGGL((k_rhs_p<DIM, NP, BLEND, false, false>), nb, bl, 0, s, a);
-        return hip_check(c, hipGetLastError(), "k_rhs_p launch");
+        if (c->geo.bcmask) return launch_points<DIM, NP, BLEND, true, false>(c, a, s);
+        return launch_points<DIM, NP, BLEND, false, false>(c, a, s);
     } else {
         if constexpr (gen_built(DIM, NP)) {
             if (c->gen) return launch_lines_sized<DIM, NP, BLEND, false, true>(c, a, s);

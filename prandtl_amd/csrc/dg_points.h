@@ -25,13 +25,13 @@ constexpr int points_epb(int TN)
     return e;
 }
 
-template <int DIM, int NP> struct PtCfg {
+template <int DIM, int NP, int FB = 0> struct PtCfg {
     static constexpr int NV = DIM + 2;
     static constexpr int K = npow(NP, DIM);
     static constexpr int NFP = npow(NP, DIM - 1);
     static constexpr int TN = DIM * K;
-    static constexpr int EPB = points_epb(TN);
-    static constexpr int BLOCK = r64(EPB * TN);
+    static constexpr int EPB = FB ? FB / TN : points_epb(TN);
+    static constexpr int BLOCK = FB ? FB : r64(EPB * TN);
     static constexpr int NR = NV + 1;   // rows: rho, v, beta, lambda
     static constexpr int KP = LnCfg<DIM, NP, 0>::KP;
     static constexpr int ES = NR * KP;
@@ -40,8 +40,9 @@ template <int DIM, int NP> struct PtCfg {
 // Whether a workgroup of one element's node threads can be launched.
 constexpr bool points_built(int DIM, int NP) { return DIM * npow(NP, DIM) <= 1024; }
 
-template <int DIM, int NP, bool BLEND, bool GEN> struct PointSmem {
-    using C = PtCfg<DIM, NP>;
+// LDS of one tile (EPB elements).
+template <int DIM, int NP, bool BLEND, int FB, bool GEN, bool AXI> struct PointSmem {
+    using C = PtCfg<DIM, NP, FB>;
     double Q[C::EPB * C::ES];                                   // rows; then the partial sums
     double X[2][BLEND ? C::EPB : 1][BLEND ? C::KP : 1];         // indicator: rho p and its transforms, in turn
     double E[BLEND ? C::EPB : 1][3][BLEND ? C::NFP : 1];        // modal energies per line
@@ -51,19 +52,25 @@ template <int DIM, int NP, bool BLEND, bool GEN> struct PointSmem {
     double Xn[NP], W[NP];                                       // LGL nodes and weights
     double D2[NP * NP];                                         // 2 D + E
     double V1[BLEND ? NP * NP : 1];                             // inverse 1-D Vandermonde
+    double R[AXI ? C::EPB : 1][AXI ? C::KP : 1];                // r of the nodes
+    double Pr[AXI ? C::EPB : 1][AXI ? C::KP : 1];               // p of the nodes
 };
 
-template <int DIM, int NP, bool BLEND, bool OPEN, bool GEN>
-__global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A)
+// One tile, as line_body: the same template parameters and arguments.
+template <int DIM, int NP, bool BLEND, bool QNS3, typename VT, int FB, bool OPEN = false, bool GEN = false,
+          bool AXI = false>
+__device__ __forceinline__ void point_body(const KArgs &A, const int tile, const int slot,
+                                           PointSmem<DIM, NP, BLEND, FB, GEN, AXI> &S)
 {
-    using C = PtCfg<DIM, NP>;
+    using C = PtCfg<DIM, NP, FB>;
     constexpr int NV = C::NV, K = C::K, NFP = C::NFP, TN = C::TN, EPB = C::EPB, BLOCK = C::BLOCK, KP = C::KP, ES = C::ES;
-    __shared__ PointSmem<DIM, NP, BLEND, GEN> S;
+    constexpr bool VISC = DIM > 1 && !AXI;   // built with viscous terms
+    static_assert(!AXI || (GEN && DIM == 2), "axisymmetric meshes are quadrilateral meshes");
     auto sQ = [&](int e2, int row, int s) -> double & { return S.Q[e2 * ES + row * KP + s]; };
 
     if (A.skip && *A.skip) return;   // uniform: before any barrier
-    const int t = threadIdx.x, slot = blockIdx.x;
-    const int ebase = xcd_remap(blockIdx.x, gridDim.x) * EPB;
+    const int t = threadIdx.x;
+    const int ebase = tile * EPB;
     const int NE = A.geo.NE;
     const size_t NK = (size_t)NE * K;
     const Phys &P = A.phys;
@@ -104,12 +111,19 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
     }
     double ys[NV];
     const size_t gi = (t < nact) ? (size_t)ebase * K + t : 0;
+    AxNode xo, xn;   // AXI: what the recoveries of the node and its neighbour load
+    size_t gt = 0;
+    if constexpr (AXI) {
+        xo = axis_load(A.y, A.geo, NK, gi);
+    } else {
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        const double y = A.y[v * NK + gi];
-        ys[v] = (t < nact) ? y : 1.0;
+        for (int v = 0; v < NV; v++) {
+            const double y = A.y[v * NK + gi];
+            ys[v] = (t < nact) ? y : 1.0;
+        }
     }
-    double pn[NV], nv[DIM], ftn[NV - 1];   // the neighbour's state, normal and viscous trace (lanes at a line's end)
+    double pn[NV], nv[DIM];   // the neighbour's state, normal and viscous trace (lanes at a line's end)
+    VT ftn[NV - 1];
     int bt = BC_PERIODIC;
     {
         size_t g = 0;
@@ -128,13 +142,18 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
             }
             g = end ? (size_t)en * K + nn : 0;
         }
+        if constexpr (AXI) {
+            xn = axis_load(A.y, A.geo, NK, g);
+            gt = g;
+        } else {
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-            const double y = A.y[v * NK + g];
-            pn[v] = end ? y : 1.0;
+            for (int v = 0; v < NV; v++) {
+                const double y = A.y[v * NK + g];
+                pn[v] = end ? y : 1.0;
+            }
         }
-        const bool vact = A.parabolic && end;
-        const double *fv = A.parabolic ? static_cast<const double *>(A.fvf) : A.y;
+        const bool vact = VISC && A.parabolic && end;
+        const VT *fv = VISC && A.parabolic ? static_cast<const VT *>(A.fvf) : reinterpret_cast<const VT *>(A.y);
         size_t on = 0;
         if (vact) {
             if constexpr (GEN) {
@@ -155,8 +174,8 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
         }
 #pragma unroll
         for (int v = 0; v < NV - 1; v++) {
-            const double b = fv[on + v * NFP];
-            ftn[v] = vact ? b : 0.0;
+            const VT b = fv[on + v * NFP];
+            ftn[v] = vact ? b : VT(0);
         }
     }
     for (int i = t; i < NP * NP; i += BLOCK) {
@@ -175,6 +194,7 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
     const int e2 = EPB == 1 ? 0 : t / K, n2 = t - e2 * K;
     const int sn = t < nact ? lines_node_slot<DIM, NP>(n2) : 0;
     if (t < nact) {
+        if constexpr (AXI) axis_state(A.y, A.geo, K, NK, gi, xo, ys);
         const NodeQ<DIM> q = node_quants<DIM>(ys, P);
         sQ(e2, 0, sn) = q.rho;
 #pragma unroll
@@ -186,6 +206,12 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
 #pragma unroll
             for (int d = 0; d < DIM; d++) vsq = (d == 0) ? q.v[d] * q.v[d] : vsq + q.v[d] * q.v[d];
             S.X[0][e2][sn] = q.rho * (P.gm1 * (ys[NV - 1] - 0.5 * q.rho * vsq));   // rho p
+        }
+        if constexpr (AXI) {
+            // PressureFromConservative (DGSEMIntegrator.cpp:1306-1315)
+            const double ke = 0.5 * ((ys[1] * ys[1] + ys[2] * ys[2]) / ys[0]);
+            S.Pr[e2][sn] = P.gm1 * (ys[3] - ke);
+            S.R[e2][sn] = A.geo.rnode[gi];
         }
         const double lq = (q.lam == q.lam) ? q.lam : 0.0;
         lam = (lam < lq) ? lq : lam;
@@ -215,6 +241,7 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
 #pragma unroll
     for (int v = 0; v < NV; v++) acc[v] = 0.0;
     if (end) {
+        if constexpr (AXI) axis_state(A.y, A.geo, K, NK, gt, xn, pn);
         const double iw0 = 1.0 / A.tab.w[0];
         double F[NV];
         if ((OPEN || GEN) && bt != BC_PERIODIC) {
@@ -247,12 +274,17 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
                 lbd = boundary_flux<DIM>(bt, r, side ? nr : -nr, nr, pn, bs, P, quirk3d, F);
             }
             lam = (lam < lbd) ? lbd : lam;
-            if (A.parabolic && (bt == BC_OUTFLOW || bt == BC_NOSLIP)) {
+            if constexpr (AXI) {
+                const double rf = S.R[el][lo];
+#pragma unroll
+                for (int v = 0; v < NV; v++) F[v] *= rf;
+            }
+            if (VISC && A.parabolic && (bt == BC_OUTFLOW || bt == BC_NOSLIP)) {
                 double fn[NV], n2q = nn[0] * nn[0];
 #pragma unroll
                 for (int d = 1; d < DIM; d++) n2q = n2q + nn[d] * nn[d];
 #pragma unroll
-                for (int v = 1; v < NV; v++) fn[v] = GEN ? ftn[v - 1] : ftn[v - 1] * (side ? nr : -nr);
+                for (int v = 1; v < NV; v++) fn[v] = GEN ? (double)ftn[v - 1] : (double)ftn[v - 1] * (side ? nr : -nr);
                 if (bt == BC_NOSLIP) {
                     double en = bs[0] * fn[1];
 #pragma unroll
@@ -267,7 +299,7 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
         } else {
             NodeQ<DIM> qo = face_node(lo), qn = node_quants<DIM>(pn, P);
             qn.ibeta = rcp_nr(qn.beta);
-            if (A.parabolic && A.quirks) {
+            if (VISC && A.parabolic && A.quirks) {
                 alias_quants<DIM>(qo, P);
                 alias_quants<DIM>(qn, P);
             }
@@ -285,10 +317,16 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
                 if (A.ec) ec_flux<DIM, false>(nvec, nr, q1, q2, P, false, F);
                 else ec_flux<DIM, true, DIM == 3>(nvec, nr, q1, q2, P, quirk3d, F);
             }
-            if (A.parabolic) {
+            if constexpr (AXI) {
+                const double rl = S.R[el][lo], rg = A.geo.rnode[gn];
+                const double rf = own ? rl : rg;
+#pragma unroll
+                for (int v = 0; v < NV; v++) F[v] *= rf;
+            }
+            if (VISC && A.parabolic) {
                 const double hn = GEN ? 0.5 : 0.5 * nr;
 #pragma unroll
-                for (int v = 1; v < NV; v++) F[v] -= ftn[v - 1] * hn;
+                for (int v = 1; v < NV; v++) F[v] -= (double)ftn[v - 1] * hn;
             }
             const double sg = own ? iw0 : -iw0;
 #pragma unroll
@@ -381,11 +419,38 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
         for (int d = 0; d < DIM; d++) nvec[d] *= om;
         const NodeQ<DIM> qa = node(lo);
         const double xa = S.Xn[m];
+        const double ra = AXI ? S.R[el][lo] : 1.0;
         auto pairs = [&](auto range) {
             constexpr int RANGE = decltype(range)::value;
 #pragma unroll
             for (int j = 1; j < NP; j++) {
                 const int b = j - 1 + (j > m ? 1 : 0);   // the j-th of the others
+                if constexpr (QNS3) {
+                    if (r == 2 && b < m) {
+                        // zeta partners b < m, as in line_body: the eta flux of
+                        // node b with node (i, NP-1, b) of its eta line
+                        if (lb < NP - 1) {
+                            const NodeQ<DIM> qz = node(slot_of(b)), qe = node(lines_slot<DIM, NP>(la, NP - 1, b));
+                            double n1[DIM], g[NV];
+                            if constexpr (GEN) {
+                                double m1[MO][DIM];
+                                line_metric<DIM>(S.Cn[el], 1, S.Xn[la], S.Xn[b], m1);
+                                const double xb = S.Xn[lb], xe = S.Xn[NP - 1];
+#pragma unroll
+                                for (int d = 0; d < DIM; d++)
+                                    n1[d] = om * (m1[0][d] + 0.5 * (xb + xe) * m1[1][d] + 0.5 * (xb * xb + xe * xe) * m1[MO - 1][d]);
+                            } else {
+#pragma unroll
+                                for (int d = 0; d < DIM; d++) n1[d] = d == 1 ? om * A.geo.nrm[1] : 0.0;
+                            }
+                            ec_flux<DIM, false>(n1, 0.0, qz, qe, P, false, g);
+                            const double d2 = S.D2[m * NP + b];
+#pragma unroll
+                            for (int v = 0; v < NV; v++) acc[v] = fma(d2, g[v], acc[v]);
+                        }
+                        continue;
+                    }
+                }
                 const NodeQ<DIM> qb = node(slot_of(b));
                 double F[NV], n[DIM];
                 if constexpr (GEN) {
@@ -396,6 +461,7 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
                     for (int d = 0; d < DIM; d++) {
                         n[d] = fma(mc[1][d], x1, mc[0][d]);
                         if constexpr (DIM == 3) n[d] = fma(mc[2][d], x2, n[d]);
+                        if constexpr (AXI) n[d] *= 0.5 * (ra + S.R[el][slot_of(b)]);
                     }
                 } else {
 #pragma unroll
@@ -408,17 +474,21 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
                 for (int v = 0; v < NV; v++) acc[v] = fma(d2, F[v], acc[v]);
             }
         };
-        double rlo = sQ(el, 0, ls[0]), rhi = rlo, blo = sQ(el, NV - 1, ls[0]), bhi = blo;
+        if constexpr (QNS3) {
+            pairs(std::integral_constant<int, LM_PAIR>{});
+        } else {
+            double rlo = sQ(el, 0, ls[0]), rhi = rlo, blo = sQ(el, NV - 1, ls[0]), bhi = blo;
 #pragma unroll
-        for (int q = 1; q < NP; q++) {
-            const double a = sQ(el, 0, ls[q]), b = sQ(el, NV - 1, ls[q]);
-            rlo = fmin(rlo, a); rhi = fmax(rhi, a);
-            blo = fmin(blo, b); bhi = fmax(bhi, b);
+            for (int q = 1; q < NP; q++) {
+                const double a = sQ(el, 0, ls[q]), b = sQ(el, NV - 1, ls[q]);
+                rlo = fmin(rlo, a); rhi = fmax(rhi, a);
+                blo = fmin(blo, b); bhi = fmax(bhi, b);
+            }
+            const double dr = rhi - rlo, rs = rhi + rlo, db = bhi - blo, bs = bhi + blo;
+            if (DIM == 3 && ((dr < 0.01 * rs) & (db < 0.01 * bs))) pairs(std::integral_constant<int, LM_SHORT>{});
+            else if (__any(lm_outside(rlo, rhi) | lm_outside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
+            else pairs(std::integral_constant<int, LM_MID>{});
         }
-        const double dr = rhi - rlo, rs = rhi + rlo, db = bhi - blo, bs = bhi + blo;
-        if (DIM == 3 && ((dr < 0.01 * rs) & (db < 0.01 * bs))) pairs(std::integral_constant<int, LM_SHORT>{});
-        else if (__any(lm_outside(rlo, rhi) | lm_outside(blo, bhi))) pairs(std::integral_constant<int, LM_ANY>{});
-        else pairs(std::integral_constant<int, LM_MID>{});
 
         if constexpr (BLEND) {
             if (alpha_e > 0.0) {
@@ -434,6 +504,12 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
 #pragma unroll
                         for (int d = 0; d < DIM; d++) ns[d] = sv[d];
                         nd = normal_length<DIM>(ns, A.geo.nsc, A.geo.insc);
+                        if constexpr (AXI) {
+                            const double rh = 0.5 * (S.R[el][slot_of(i)] + S.R[el][slot_of(i + 1)]);
+                            nd *= rh;
+#pragma unroll
+                            for (int d = 0; d < DIM; d++) ns[d] *= rh;
+                        }
                     } else {
                         nd = A.tab.subn[0][0];
 #pragma unroll
@@ -462,7 +538,8 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
 #pragma unroll
     for (int v = 0; v < NV; v++) {
         u0v[v] = (A.mode == 2 && in) ? A.u0[v * NK + gi] : 0.0;
-        if (v > 0) vs[v - 1] = (A.parabolic && in) ? static_cast<const double *>(A.visc)[(v - 1) * NK + gi] : 0.0;
+        if constexpr (AXI) ys[v] = (A.mode != 0 && in) ? A.y[v * NK + gi] : 0.0;   // r U
+        if (v > 0) vs[v - 1] = (VISC && A.parabolic && in) ? (double)static_cast<const VT *>(A.visc)[(v - 1) * NK + gi] : 0.0;
     }
     __syncthreads();   // the partial sums take the rows' place
 #pragma unroll
@@ -479,6 +556,14 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
             double tot = -sQ(e2, v, sn);
             if (v > 0) tot += vs[v - 1];
             tot *= iJ;
+            if constexpr (AXI) {
+                if (v == 2) {
+                    // pressure source and ZeroAxisRadialMom, as in line_body
+                    tot += S.Pr[e2][sn];
+                    const int ax = A.geo.axm[gi];
+                    if (ax >= 0 && (ax & 1)) tot = 0.0;
+                }
+            }
             double o = tot;
             if (A.mode != 0) {
                 o = fma(dt, tot, ys[v]);
@@ -488,6 +573,13 @@ __global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A
         }
     }
     block_lam_max<BLOCK>(lam, lam_old, A.lam, S.Red, slot);
+}
+
+template <int DIM, int NP, bool BLEND, bool QNS3, typename VT, bool OPEN, bool GEN, bool AXI = false>
+__global__ void __launch_bounds__((PtCfg<DIM, NP>::BLOCK)) k_rhs_p(const KArgs A)
+{
+    __shared__ PointSmem<DIM, NP, BLEND, 0, GEN, AXI> S;
+    point_body<DIM, NP, BLEND, QNS3, VT, 0, OPEN, GEN, AXI>(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.x, S);
 }
 
 } // namespace prandtl
