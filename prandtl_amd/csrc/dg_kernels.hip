@@ -78,6 +78,39 @@ k_ens(const KArgs *__restrict__ cases, const EnsTile *__restrict__ tiles)
     }
 }
 
+// The same with node threads (dg_points.h), for ensembles that do not fill the
+// chip with line threads; bitwise equal.  The workgroup is that of the largest
+// tile that a 2-D order's node threads need.
+constexpr int ENS_PBLOCK = 256;
+
+template <int NP, bool BLEND> constexpr size_t ens_psmem() { return sizeof(PointSmem<2, NP, BLEND, ENS_PBLOCK, false, false>); }
+constexpr size_t ENS_PSMEM = cmax(cmax(cmax(ens_psmem<3, false>(), ens_psmem<3, true>()), cmax(ens_psmem<4, false>(), ens_psmem<4, true>())),
+                                  cmax(cmax(ens_psmem<5, false>(), ens_psmem<5, true>()), cmax(ens_psmem<6, false>(), ens_psmem<6, true>())));
+
+template <int NP, bool BLEND> __device__ __forceinline__ void ens_ptile(const KArgs &A, int g, double *smem)
+{
+    point_body<2, NP, BLEND, false, double, ENS_PBLOCK>(
+        A, g, g, *reinterpret_cast<PointSmem<2, NP, BLEND, ENS_PBLOCK, false, false> *>(smem));
+}
+
+__global__ void __launch_bounds__(ENS_PBLOCK) k_ens_p(const KArgs *__restrict__ cases, const EnsTile *__restrict__ tiles)
+{
+    __shared__ __align__(16) double smem[(ENS_PSMEM + 7) / 8];
+    const EnsTile T = tiles[blockIdx.x];
+    const KArgs &A = cases[T.c];
+    switch (T.v) {
+    case 0: ens_ptile<3, false>(A, T.g, smem); break;
+    case 1: ens_ptile<3, true>(A, T.g, smem); break;
+    case 2: ens_ptile<4, false>(A, T.g, smem); break;
+    case 3: ens_ptile<4, true>(A, T.g, smem); break;
+    case 4: ens_ptile<5, false>(A, T.g, smem); break;
+    case 5: ens_ptile<5, true>(A, T.g, smem); break;
+    case 6: ens_ptile<6, false>(A, T.g, smem); break;
+    case 7: ens_ptile<6, true>(A, T.g, smem); break;
+    default: break;
+    }
+}
+
 // Persistent form: a fixed grid (a chosen number of workgroups per CU) loops
 // over the same cost-sorted tile list, each workgroup taking the next tile
 // from a device counter until the list is exhausted (every workgroup leaves
@@ -1682,8 +1715,10 @@ struct prandtl_ensemble {
     std::vector<double *> u;               // caller state pointers the arguments were built for
     std::vector<double> dt;                // step sizes last copied to d_dts
     KArgs *d_args[3] = {nullptr, nullptr, nullptr};
-    EnsTile *d_tiles = nullptr;
+    EnsTile *d_tiles = nullptr;    // of line threads
     int ntiles = 0;
+    EnsTile *d_ptiles = nullptr;   // of node threads (mode 0 of small ensembles), else null
+    int nptiles = 0;
     double *d_dts = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1697,20 +1732,25 @@ struct prandtl_ensemble {
 
 namespace {
 
-int ens_epb(int NP, int blend)
+// elements per tile, of line threads and of node threads
+int ens_epb(int NP)
 {
-    switch (NP * 2 + blend) {
-    case 6: return LnCfg<2, 3>::EPB;
-    case 7: return LnCfg<2, 3>::EPB;
-    case 8: return LnCfg<2, 4>::EPB;
-    case 9: return LnCfg<2, 4>::EPB;
-    case 10: return LnCfg<2, 5>::EPB;
-    case 11: return LnCfg<2, 5>::EPB;
-    case 12: return LnCfg<2, 6>::EPB;
-    case 13: return LnCfg<2, 6>::EPB;
+    switch (NP) {
+    case 3: return LnCfg<2, 3>::EPB;
+    case 4: return LnCfg<2, 4>::EPB;
+    case 5: return LnCfg<2, 5>::EPB;
+    case 6: return LnCfg<2, 6>::EPB;
     default: return 0;
     }
 }
+int ens_pepb(int NP) { return ENS_PBLOCK / (2 * NP * NP); }
+
+// Node-thread workgroups of one order up to which an ensemble of it takes them
+// (of several orders: while the shares add up to less than 1).  us per step, line
+// / node threads: N = 2 4 x 32^2 30.5 / 30.0, 8 x 32^2 35.1 / 36.4; N = 3 4 x 32^2 32.8 /
+// 30.2, 8 x 32^2 38.9 / 42.5; N = 4 48^2 34.9 / 31.8, 4 x 32^2 42.6 / 45.4; N = 5 blended
+// 8 x 16^2 51.9 / 45.8, 48^2 46.4 / 41.9, 4 x 32^2 54.5 / 66.2.
+int ens_points_max(int NP) { return NP == 3 ? 448 : NP == 4 ? 512 : NP == 5 ? 640 : 800; }
 
 // relative cost of one tile of variant v = 2*(NP-3) + blend: nodes per tile
 // times the per-node pair work (NP-1 partners per direction) plus the
@@ -1718,7 +1758,7 @@ int ens_epb(int NP, int blend)
 double ens_cost(int v)
 {
     const int NP = 3 + v / 2, blend = v & 1;
-    const int epb = ens_epb(NP, blend);
+    const int epb = ens_epb(NP);
     return (double)epb * NP * NP * ((NP - 1) + 4.0 + (blend ? 3.0 : 0.0));
 }
 
@@ -1759,7 +1799,9 @@ int ens_bind(prandtl_ensemble *E, double *const *u, hipStream_t s)
 // one stage k of every case in the current launch form
 void ens_stage(prandtl_ensemble *E, int k, int mode, hipStream_t s)
 {
-    if (mode == 0)
+    if (mode == 0 && E->d_ptiles)
+        hipLaunchKernelGGL(k_ens_p, dim3(E->nptiles), dim3(ENS_PBLOCK), 0, s, E->d_args[k], E->d_ptiles);
+    else if (mode == 0)
         hipLaunchKernelGGL(k_ens, dim3(E->ntiles), dim3(ENS_BLOCK), 0, s, E->d_args[k], E->d_tiles);
     else
         hipLaunchKernelGGL(k_ens_q, dim3(4 * mode * E->ncu), dim3(ENS_BLOCK), 0, s, E->d_args[k], E->d_tiles, E->ntiles,
@@ -1795,7 +1837,8 @@ int prandtl_ensemble_create(int ncases, const prandtl_mesh_desc *meshes, const p
     prandtl_ensemble *E = new (std::nothrow) prandtl_ensemble();
     if (!E) return ens_fail(nullptr, PRANDTL_ERR_NOMEM, "host allocation");
     E->n = ncases;
-    std::vector<EnsTile> tiles;
+    std::vector<EnsTile> tiles, ptiles;
+    double share = 0.0;
     for (int i = 0; i < ncases; i++) {
         prandtl_ctx *c = nullptr;
         const int rc = prandtl_create(&meshes[i], &params[i], &c);
@@ -1805,15 +1848,21 @@ int prandtl_ensemble_create(int ncases, const prandtl_mesh_desc *meshes, const p
         }
         E->ctx.push_back(c);
         const int blend = params[i].blending ? 1 : 0;
-        const int epb = ens_epb(c->Np, blend);
-        const int groups = (c->NE + epb - 1) / epb;
-        for (int g = 0; g < groups; g++) tiles.push_back({i, g, 2 * (c->Np - 3) + blend});
+        auto add = [&](std::vector<EnsTile> &to, int epb) {
+            for (int g = 0; g < (c->NE + epb - 1) / epb; g++) to.push_back({i, g, 2 * (c->Np - 3) + blend});
+        };
+        add(tiles, ens_epb(c->Np));
+        add(ptiles, ens_pepb(c->Np));
+        share += (double)((c->NE + ens_pepb(c->Np) - 1) / ens_pepb(c->Np)) / ens_points_max(c->Np);
     }
+    if (share > 1.0) ptiles.clear();
     // most expensive tiles first, so the tail of the dispatch order is made of
     // cheap tiles (longest-processing-time-first list scheduling)
-    std::stable_sort(tiles.begin(), tiles.end(),
-                     [](const EnsTile &a, const EnsTile &b) { return ens_cost(a.v) > ens_cost(b.v); });
+    for (auto *t : {&tiles, &ptiles})
+        std::stable_sort(t->begin(), t->end(),
+                         [](const EnsTile &a, const EnsTile &b) { return ens_cost(a.v) > ens_cost(b.v); });
     E->ntiles = (int)tiles.size();
+    E->nptiles = (int)ptiles.size();
     hipError_t e = hipSuccess;
     for (int k = 0; k < 3 && e == hipSuccess; k++) e = hipMalloc(&E->d_args[k], sizeof(KArgs) * ncases);
     if (e == hipSuccess) e = hipMalloc(&E->d_tiles, sizeof(EnsTile) * E->ntiles);
@@ -1825,6 +1874,10 @@ int prandtl_ensemble_create(int ncases, const prandtl_mesh_desc *meshes, const p
         if (e == hipSuccess) e = hipDeviceGetAttribute(&E->ncu, hipDeviceAttributeMultiprocessorCount, dev);
     }
     if (e == hipSuccess) e = hipMemcpy(E->d_tiles, tiles.data(), sizeof(EnsTile) * E->ntiles, hipMemcpyHostToDevice);
+    if (e == hipSuccess && E->nptiles) {
+        e = hipMalloc(&E->d_ptiles, sizeof(EnsTile) * E->nptiles);
+        if (e == hipSuccess) e = hipMemcpy(E->d_ptiles, ptiles.data(), sizeof(EnsTile) * E->nptiles, hipMemcpyHostToDevice);
+    }
     if (e != hipSuccess) {
         g_create_err = std::string("ensemble device allocation: ") + hipGetErrorString(e);
         prandtl_ensemble_destroy(E);
@@ -1842,6 +1895,7 @@ void prandtl_ensemble_destroy(prandtl_ensemble *E)
     for (int k = 0; k < 3; k++)
         if (E->d_args[k]) (void)hipFree(E->d_args[k]);
     if (E->d_tiles) (void)hipFree(E->d_tiles);
+    if (E->d_ptiles) (void)hipFree(E->d_ptiles);
     if (E->d_dts) (void)hipFree(E->d_dts);
     if (E->d_counters) (void)hipFree(E->d_counters);
     for (prandtl_ctx *c : E->ctx) prandtl_destroy(c);
