@@ -131,9 +131,10 @@ template <int DIM, int NP, int FB, bool OPEN> void launch_visc_l(prandtl_ctx *c,
 // over more of them.  Euler right-hand sides, natural against this: 3-D N = 3
 // 512 elements 9.3 -> 8.0 us (2,197 elements 15.7 against 14.0, 4,096 18.6
 // against 18.7), N = 4 252 elements 10.8 -> 8.9, N = 2 125 elements 10.7 -> 8.5.
-// At N = 2, whose natural workgroup holds 9 elements, a single wave of 2 is
-// better up to 13,824 elements (4,096: RHS 11.5 -> 9.8, k_visc_l 9.5 -> 8.3;
-// 13,824: 23.0 -> 22.4, 18.5 both; 62,320: 87 against 89, 57 against 59).
+// At N = 2, whose natural workgroup holds 7 elements, a single wave of 2 is
+// better up to 13,824 elements: 4,096 RHS 11.5 -> 9.8, k_visc_l 9.5 -> 8.3; right-
+// hand sides at 13,800 Euler 21.4 -> 21.1, blended 32.4 -> 31.3, mixed 36.0 -> 35.5,
+// hexahedra 29.5 and 29.6; at 17,550 25.4 against 25.8, 45.8 against 46.7.
 // Not the faithful NS-3D form at N = 4, whose small workgroup fills 75 of 128
 // threads: 720 elements 27.7 -> 25.6, walls 32.8 -> 30.1, hexahedra 35.2 -> 33.6.
 inline bool qns3(const prandtl_ctx *c) { return c->dim == 3 && c->prm.parabolic && c->prm.quirks; }
@@ -141,7 +142,8 @@ constexpr int lines_small_fb(int DIM, int NP) { return DIM != 3 || NP > 6 ? 0 : 
 template <int DIM, int NP> bool lines_small(const prandtl_ctx *c)
 {
     if (NP == 5 && qns3(c)) return false;
-    return lines_small_fb(DIM, NP) > 0 && c->NE < (NP == 3 ? 1536 : 256) * LnCfg<DIM, NP>::EPB;
+    if (DIM == 3 && NP == 3) return c->NE <= 13824;
+    return lines_small_fb(DIM, NP) > 0 && c->NE < 256 * LnCfg<DIM, NP>::EPB;
 }
 
 // Orders the general-geometry kernels are built for: 2-D N = 1..5, 3-D N = 2..4.

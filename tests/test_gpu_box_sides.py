@@ -18,10 +18,10 @@ TOL = 1e-12
 G = 1.4
 NS = dict(parabolic=True, mu=0.02, Pr=0.71)
 
-# 3-D: node threads up to 341, 256 and 232 elements at N = 3, 4, 5 (N = 2 only
-# with blending, up to 248 of 2 a workgroup), the small workgroup up to 1023,
-# 767 and 511, at N = 2 up to 10,752 or 13,824; 2-D: node threads up to 3,072
-# waves at most
+# 3-D: node threads up to 341, 256 and 232 elements at N = 3, 4, 5 (faithful
+# Navier-Stokes 768 and 554 at N = 3, 4; N = 2 only with blending), the small
+# workgroup up to 1023, 767 and 511, at N = 2 up to 13,824; 2-D: node threads up
+# to 6,144, 5,376, 4,096 and 2,496 elements at most
 SIZES = {2: {2: [(5, 4), (90, 91)], 3: [(5, 4), (80, 81)], 4: [(5, 4), (66, 67)], 5: [(5, 4), (61, 60)]},
          3: {2: [(3, 4, 5), (9, 9, 8), (24, 24, 25)], 3: [(3, 4, 5), (8, 8, 7), (11, 10, 10)],
              4: [(3, 4, 5), (7, 8, 7), (10, 9, 9)], 5: [(3, 4, 5), (7, 7, 7), (9, 8, 8)],
