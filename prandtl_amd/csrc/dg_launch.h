@@ -357,9 +357,9 @@ int launch_rhs_t(prandtl_ctx *c, const KArgs &a, hipStream_t s)
             if (c->gen) return launch_lines_sized<DIM, NP, BLEND, false, true>(c, a, s);
         }
         if (c->geo.bcmask) return launch_lines_sized<DIM, NP, BLEND, true, false>(c, a, s);
-        // forced shapes (a 2-D tile of 64 threads is the natural one)
-        if constexpr (DIM == 3 && rhs_shape_ok(DIM, NP, BLEND, 1))
-            if (c->rhs_shape == 1) return launch_lines<DIM, NP, BLEND, 64, false, false>(c, a, s);
+        // forced shapes: line threads (64 is the natural size in 2-D)
+        if constexpr (rhs_shape_ok(DIM, NP, BLEND, 1))
+            if (c->rhs_shape == 1) return launch_lines<DIM, NP, BLEND, DIM == 2 ? 0 : 64, false, false>(c, a, s);
         if constexpr (rhs_shape_ok(DIM, NP, BLEND, 2))
             if (c->rhs_shape == 2) return launch_lines<DIM, NP, BLEND, 128, false, false>(c, a, s);
         if constexpr (rhs_shape_ok(DIM, NP, BLEND, 3))
