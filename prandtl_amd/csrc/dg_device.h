@@ -85,8 +85,8 @@ struct Geo {
     const double *bfn;    // null, or per attribute [16]: a split outer state [kind, n0, n1, n2,
                           // offset, speed, below[5], above[5]] (0 kind: the constant state)
     const double *subn;   // [NE][2][NFP][NP-1][2] subcell interface normals
-    const double *corner; // hexahedral meshes: [NE][8][3] element corners; the per-node metrics
-                          // are recomputed from them (met and jac are not stored)
+    const double *corner; // [NE][4][2] or [NE][8][3] element corners: the RHS forms its metrics from
+                          // them, in 3-D k_visc too (met is not stored there)
     // axisymmetric quadrilateral meshes (null otherwise)
     const double *rnode;  // [NE*K] r = y of each node
     const int *axm;       // [NE*K] -1 off the axis, else 2 d + (1: radial RHS zeroed), d the descriptor
@@ -139,7 +139,6 @@ struct VArgs {
 };
 
 constexpr int cmx(int a, int b) { return a > b ? a : b; }
-constexpr int pow2_at_least(int x) { return x <= 1 ? 1 : 2 * pow2_at_least((x + 1) / 2); }
 constexpr int r64(int x) { return ((x + 63) / 64) * 64; }
 // NP^d: nodes per element (d = DIM) and per face (d = DIM - 1)
 constexpr int npow(int NP, int d) { return d <= 0 ? 1 : NP * npow(NP, d - 1); }
@@ -178,7 +177,6 @@ template <int DIM, int NP, int FB = 0> struct VCfg {
 template <int DIM, int NP>
 __device__ __forceinline__ int line_node(int r, int l, int m)
 {
-    if (DIM == 1) return m;
     if (DIM == 2) return r == 0 ? l * NP + m : m * NP + l;
     const int a = l % NP, b = l / NP;
     if (r == 0) return (b * NP + a) * NP + m;
@@ -189,7 +187,6 @@ __device__ __forceinline__ int line_node(int r, int l, int m)
 template <int DIM, int NP>
 __device__ __forceinline__ int line_of(int r, int i, int j, int k)
 {
-    if (DIM == 1) return 0;
     if (DIM == 2) return r == 0 ? j : i;
     if (r == 0) return k * NP + j;
     if (r == 1) return k * NP + i;
@@ -321,9 +318,10 @@ __device__ __forceinline__ void block_lam_max(double lam, double old, double *sl
 }
 
 // Launch shapes of the RHS in two and three dimensions: which workgroup sizes
-// a caller may force (PRANDTL_SHAPES).  A shape is offered where a workgroup
-// of its size holds an element's nodes one per thread and differs from the
-// size rshape() gives as the natural one.
+// a caller may force (PRANDTL_SHAPES).  The set is part of the interface, callers
+// keep shapes that autotune found: it is that of workgroups with a thread for each
+// of an element's nodes and pairs' jobs (rshape), other than the one that was the
+// natural one for those.  Every size in it holds an element's lines.
 struct RShape {
     int K, WORK, EPB, BLOCK;
 };

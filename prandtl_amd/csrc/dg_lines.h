@@ -140,21 +140,20 @@ template <int DIM, int NP, int FB> struct LinePos {
         } else {
             el = C::EPB == 1 ? 0 : t / TE;
             rem = t - el * TE;
-            r = DIM == 1 ? 0 : rem / NFP;
+            r = rem / NFP;
             if constexpr (NFP == 64 && C::EPB == 1) r = __builtin_amdgcn_readfirstlane(r);
             l = rem - r * NFP;
         }
         la = DIM == 3 ? l % NP : l;
         lb = DIM == 3 ? l / NP : 0;
-        base = DIM == 1 ? 0 : r == 0 ? l * NP : (DIM == 3 && r == 1 ? lb * NP * NP + la : l);
+        base = r == 0 ? l * NP : (DIM == 3 && r == 1 ? lb * NP * NP + la : l);
         stride = r == 0 ? 1 : (r == 1 ? NP : NP * NP);
     }
     __device__ __forceinline__ void slots(int *ls) const
     {
 #pragma unroll
         for (int m = 0; m < NP; m++) {
-            if constexpr (DIM == 1) ls[m] = m;
-            else if constexpr (DIM == 2) ls[m] = r == 0 ? lines_slot<DIM, NP>(m, la, 0) : lines_slot<DIM, NP>(la, m, 0);
+            if constexpr (DIM == 2) ls[m] = r == 0 ? lines_slot<DIM, NP>(m, la, 0) : lines_slot<DIM, NP>(la, m, 0);
             else ls[m] = lines_slot<DIM, NP>(r == 0 ? m : la, r == 1 ? m : (r == 0 ? la : lb), r == 2 ? m : lb);
         }
     }
@@ -273,6 +272,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
     constexpr int NV = C::NV, K = C::K, NFP = C::NFP, TE = C::TE, EPB = C::EPB, BLOCK = C::BLOCK, NPASS = C::NPASS;
     constexpr int KP = C::KP, ES = C::ES;
     constexpr bool LTAB = lines_ltab(DIM, NP, BLEND);
+    static_assert(DIM > 1, "1-D right-hand sides run node threads");
     static_assert(!AXI || (GEN && DIM == 2), "axisymmetric meshes are quadrilateral meshes");
     auto sQ = [&](int e2, int row, int s) -> double & { return S.Q[e2 * ES + row * KP + s]; };
 
@@ -357,7 +357,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
                 pt[side][v] = lact ? y : 1.0;
             }
         }
-        if constexpr (DIM > 1 && !AXI) {
+        if constexpr (!AXI) {
             // the neighbour's viscous face trace (this element's own is in
             // k_visc's volume term); without viscous terms it is read from
             // the state array and discarded.  On a boundary side: this
@@ -528,7 +528,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
 #pragma unroll
                     for (int v = 0; v < NV; v++) F[v] *= rf;
                 }
-                if constexpr (DIM > 1 && !AXI) {
+                if constexpr (!AXI) {
                     if (A.parabolic && (bt[side] == BC_OUTFLOW || bt[side] == BC_NOSLIP)) {
                         // - Fv.n of the interior state and gradients; inflow
                         // and specified states have zero gradients, so no
@@ -555,7 +555,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
             }
             NodeQ<DIM> qo = face_node(mo), qn = node_quants<DIM>(pn, P);
             qn.ibeta = rcp_nr(qn.beta);
-            if constexpr (DIM > 1 && !AXI) {
+            if constexpr (!AXI) {
                 if (A.parabolic && A.quirks) {
                     alias_quants<DIM>(qo, P);
                     alias_quants<DIM>(qn, P);
@@ -584,7 +584,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
 #pragma unroll
                 for (int v = 0; v < NV; v++) F[v] *= rf;
             }
-            if constexpr (DIM > 1 && !AXI) {
+            if constexpr (!AXI) {
                 if (A.parabolic) {
                     // the neighbour's half of the mean of the two sides' traces
                     // Fv.n (boxes: per unit normal)
@@ -632,8 +632,8 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
 #pragma unroll
                     for (int a = 0; a < NP - 2; a++) lo = fma(md[a], md[a], lo);
                     const double mid = md[NP - 2] * md[NP - 2], top = md[NP - 1] * md[NP - 1];
-                    const bool in1 = (DIM == 1 || la <= NP - 2) && lb <= NP - 2;
-                    const bool in2 = NP > 2 && (DIM == 1 || la <= NP - 3) && (DIM < 3 || lb <= NP - 3);
+                    const bool in1 = la <= NP - 2 && lb <= NP - 2;
+                    const bool in2 = NP > 2 && la <= NP - 3 && (DIM < 3 || lb <= NP - 3);
                     S.E[el][0][l] = in1 ? top : lo + mid + top;
                     S.E[el][1][l] = in2 ? mid : (in1 ? lo + mid : 0.0);
                     S.E[el][2][l] = in2 ? lo : 0.0;
@@ -874,7 +874,7 @@ __device__ __forceinline__ void line_body(const KArgs &A, const int tile, const 
         for (int v = 0; v < NV; v++) {
             y[v] = (A.mode != 0 && in) ? A.y[v * NK + gi] : 0.0;
             u0[v] = (A.mode == 2 && in) ? A.u0[v * NK + gi] : 0.0;
-            if (v > 0) vi[v - 1] = (DIM > 1 && A.parabolic && in) ? (double)static_cast<const VT *>(A.visc)[(v - 1) * NK + gi] : 0.0;
+            if (v > 0) vi[v - 1] = (A.parabolic && in) ? (double)static_cast<const VT *>(A.visc)[(v - 1) * NK + gi] : 0.0;
         }
     };
     if constexpr (PRE) {
