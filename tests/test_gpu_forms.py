@@ -106,7 +106,7 @@ def test_hexahedra(cuda, order, n, form):
 
 # (order, one period, its repetitions along x): the period by node threads, the
 # whole by line threads
-REPEAT = [(2, (8, 4), 256), (3, (8, 4), 160), (4, (8, 4), 128), (5, (8, 4), 96), (2, (2, 4, 2), 128), (3, (2, 4, 2), 64),
+REPEAT = [(2, (8, 4), 256), (3, (8, 4), 160), (4, (8, 4), 128), (5, (8, 4), 96), (2, (2, 4, 2), 128), (2, (2, 4, 2), 1024), (3, (2, 4, 2), 64),
           (4, (2, 4, 2), 64), (5, (2, 4, 2), 32)]
 
 

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("walls", [False, True])
-@pytest.mark.parametrize("order,nelem", [(2, (70, 71)), (3, (60, 61)), (4, (50, 51)), (5, (45, 44)), (2, (16, 15, 17)),
+@pytest.mark.parametrize("order,nelem", [(2, (70, 71)), (3, (60, 61)), (4, (50, 51)), (5, (45, 44)), (2, (16, 15, 17)), (2, (24, 24, 25)),
                                          (3, (11, 12, 10)), (4, (9, 10, 9)), (5, (8, 8, 9)), (6, (6, 5, 6)), (7, (5, 4, 5))])
 def test_viscous_error(cuda, order, nelem, walls):
     import torch
