@@ -7,7 +7,7 @@ plain FP64.  A "step" is one SSP-RK3 step = three RHS evaluations with the
 stage combinations fused in; DOF-updates/s = nodes x RHS evaluations / s.
 
 The state is resident in HBM before the timed region starts.  The JSON line
-also carries the roofline of the dominant kernel (k_rhs, timed with HIP
+also carries the roofline of the dominant kernel (the right-hand side's, timed with HIP
 events on its own stream inside the timed region) and a CPU baseline: the
 oracle (an FP64 CPU restatement of the reference RHS, not MFEM) timed on this
 host on a bounded sample.
@@ -610,14 +610,14 @@ def main():
     alpha, _ = op.alpha()
     blend_frac = float((alpha > 0).mean()) if cfg.get("blending") else 0.0
     fl_rhs = (counts["volume"] + counts["surface"] + counts["fv"] * blend_frac + counts["indicator"]
-              + counts["assembly"] + 4 * nv)          # k_rhs, with the RK stage combination
-    fl_visc = counts["lifting"] + counts["viscous"]    # k_visc
+              + counts["assembly"] + 4 * nv)          # the RHS kernel, with the RK stage combination
+    fl_visc = counts["lifting"] + counts["viscous"]    # the viscous kernel
     # Compulsory HBM bytes per node of one RHS + RK stage: read the stage
     # state, read u^n on two stages of three, write the stage output.  The
     # viscous intermediates and geometry tables are implementation bytes
     # (measured, in "traffic").
     by_node = 8 * nv * (1 + 1 + 2.0 / 3.0)
-    kname = "k_rhs<%d,%d>" % (cfg["dim"], cfg["order"] + 1)
+    kname = "rhs<%d,%d>" % (cfg["dim"], cfg["order"] + 1)   # by dimension and nodes per direction
     traffic = measured_traffic(name, kname) if (args.precision == "fp64" and not quirks) else None
     roof = with_measured(roofline(fl_rhs * nodes, by_node * nodes, t_rhs, kname, traffic), peaks)
     t_visc = ms_visc / max(n_visc, 1) * 1e-3
@@ -625,7 +625,7 @@ def main():
                        "tflops": fl_rhs * nodes / t_rhs / 1e12,
                        "frac_fp64": fl_rhs * nodes / t_rhs / PEAK_FP64}}
     if n_visc:
-        vname = "k_visc<%d,%d>" % (cfg["dim"], cfg["order"] + 1)
+        vname = "visc<%d,%d>" % (cfg["dim"], cfg["order"] + 1)
         kernels[vname] = {"avg_launch_us": t_visc * 1e6, "flops_per_node": fl_visc,
                           "tflops": fl_visc * nodes / t_visc / 1e12,
                           "frac_fp64": fl_visc * nodes / t_visc / PEAK_FP64,
@@ -658,7 +658,7 @@ def main():
                    "rhs_per_step": 3, "dt": dt, "state_ok": bool(ok), "hip_graph": True,
                    "launch_shapes": shape, "launch_shape_us": shape_us,
                    "ms_per_step_event_profiled": elapsed_prof / psteps * 1e3,
-                   "kernel_ms": {"k_rhs": ms_rhs / max(n_rhs, 1), "k_visc": ms_visc / max(n_visc, 1)},
+                   "kernel_ms": {"rhs": ms_rhs / max(n_rhs, 1), "visc": ms_visc / max(n_visc, 1)},
                    "kernels": kernels, "rhs_roofline": whole, "measured_peaks": peaks},
         "roofline": roof,
     }
