@@ -229,7 +229,7 @@ int prandtl_rhs(prandtl_ctx *ctx, const double *u_dev, double *dudt_dev, void *s
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  It takes no context: the operator's tables are built on
  * the host at each call and passed to the kernels by value, and the kernels'
- * scratch (k_visc's viscous sums and face traces, the wave-speed slots,
+ * scratch (the viscous kernel's sums and face traces, the wave-speed slots,
  * alpha, eta, the box's boundary states) lives in a fixed 32 MiB device array
  * of the library, one per GPU, held until the process ends.  The call makes
  * no hipMalloc, hipFree or other allocating call on the device; it returns
@@ -254,8 +254,11 @@ int prandtl_rk3_step(prandtl_ctx *ctx, double *u_dev, double dt, void *stream);
  * from the running maximum wave speed, set after an initial RHS evaluation
  * and after every step; otherwise the fixed step dt.  Stops when
  * t >= t_final - 1e-8 dt, or after max_steps steps if max_steps > 0.  No host
- * synchronisation per step: batches of 16 steps run from one graph (on a
- * non-null stream) and the host reads the loop state once per batch; steps
+ * synchronisation per step: steps are enqueued in chunks of 8, two chunks in
+ * flight, and the host reads the loop state after one while the next runs; on
+ * a non-null stream a loop with 64 or more steps to go replays a chunk as a
+ * graph, captured while the first ones run.  At most max_steps steps are
+ * enqueued; steps
  * after the end do nothing.  *t_io receives the final time, *steps_out
  * (may be NULL) the number of steps.  Bitwise the same steps as the host
  * loop of prandtl_rk3_step and prandtl_max_wave_speed.  check_every > 0:
@@ -275,24 +278,24 @@ int prandtl_set_graph(prandtl_ctx *ctx, int enable);
  * workgroup of a kernel takes and how many threads it has.  kernel is
  * PRANDTL_KERNEL_RHS (the flux-differencing kernel) or PRANDTL_KERNEL_VISC
  * (the BR1 lifting and viscous-flux kernel, Navier-Stokes only).  Shape 0 is
- * the default; shapes 1..3 force 64, 128 or 256 threads per workgroup where
- * that still gives every node its own thread.  Every shape gives bitwise the
- * same results.  PRANDTL_ERR_UNSUPPORTED for a shape this case does not
- * have. */
+ * the default, chosen by the mesh's size; shapes 1..3 force 64, 128 or 256
+ * threads per workgroup (of line threads in the RHS), offered where those are
+ * at least an element's nodes.  Every shape gives bitwise the same results.
+ * PRANDTL_ERR_UNSUPPORTED for a shape this case does not have. */
 #define PRANDTL_SHAPES 4
 #define PRANDTL_KERNEL_RHS 0
 #define PRANDTL_KERNEL_VISC 1
 int prandtl_set_shape(prandtl_ctx *ctx, int kernel, int shape);
 
 /* Kernel algorithm of the flux-differencing RHS (no counterpart in the
- * reference; the operator is the same, DGSEMIntegrator.cpp:151-1196).  Every
- * 2-D and 3-D mesh runs k_rhs_l, one thread per tensor line.  Periodic
- * Cartesian boxes in 3-D, N = 2..4, have two settings that run the same
- * kernels: PRANDTL_ALGO_LINE (the default at N = 2 and 3 and, with blending,
- * at N = 4) has launch shape 0 only (both kernels in the mixed form at N = 3,
- * else the RHS kernel), PRANDTL_ALGO_TILE the forced launch shapes.  Their
- * results are the
- * same.  Every other context reports PRANDTL_ALGO_TILE, and
+ * reference; the operator is the same, DGSEMIntegrator.cpp:151-1196).  Meshes
+ * run k_rhs_l, one thread per tensor line, or, in 1-D and where a mesh is too
+ * small for that, k_rhs_p, one thread per node and direction; their results are
+ * equal bit for bit.  Periodic Cartesian boxes in 3-D, N = 2..4, have two
+ * settings that run the same kernels: PRANDTL_ALGO_LINE (the default at N = 2 and
+ * 3 and, with blending, at N = 4) has launch shape 0 only (both kernels in the
+ * mixed form at N = 3, else the RHS kernel), PRANDTL_ALGO_TILE the forced launch
+ * shapes.  Every other context reports PRANDTL_ALGO_TILE, and
  * PRANDTL_ERR_UNSUPPORTED for PRANDTL_ALGO_LINE. */
 #define PRANDTL_ALGO_TILE 0
 #define PRANDTL_ALGO_LINE 1
@@ -434,9 +437,10 @@ const char *prandtl_ensemble_last_error(const prandtl_ensemble *ens);
 
 /* Launch form of the ensemble's stages (no counterpart in the reference):
  * mode 0 launches one workgroup per element tile (the cost-sorted tile list
- * is the dispatch order); mode g = 1..PRANDTL_ENS_MAX_PER_CU launches 4 g
- * persistent workgroups of one wave per CU that take tiles from a device counter until
- * the list is exhausted.  Every form gives bitwise the same results. */
+ * is the dispatch order; tiles of node threads where the ensemble is too small
+ * for line threads); mode g = 1..PRANDTL_ENS_MAX_PER_CU launches 4 g persistent
+ * workgroups of one wave per CU that take tiles of line threads from a device
+ * counter until the list is exhausted.  Every form gives bitwise the same results. */
 #define PRANDTL_ENS_MAX_PER_CU 4
 int prandtl_ensemble_set_mode(prandtl_ensemble *ens, int mode);
 /* Autotuner of the launch form: binds u_dev / dt as prandtl_ensemble_rk3_step
