@@ -1,12 +1,12 @@
 // Host unit of libprandtl_hip.so: the C ABI of include/prandtl_hip.h
 // (contexts, RHS and RK3 entry points, hipGraph capture, autotuner, device
 // time loop, checkpoints, primitives) plus the small utility kernels and
-// k_ens, the batched-ensemble kernel.
+// the batched ensemble's kernels (k_ens, k_ens_p, k_ens_q).
 //
-// The DGSEM kernels themselves are templates in
-// dg_device.h; their launch code (dg_launch.h) is instantiated per
-// (dimension, order) in inst.hip, and this unit calls those instances
-// through the PRANDTL_DISPATCH switch below.
+// The DGSEM kernels themselves are templates in dg_lines.h, dg_points.h,
+// dg_visc_lines.h and dg_device.h; their launch code (dg_launch.h) is
+// instantiated per (dimension, order) in inst.hip, and this unit calls those
+// instances through the PRANDTL_DISPATCH switch below.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -1235,7 +1235,7 @@ int prandtl_autotune(prandtl_ctx *c, const double *u, int *shapes_out, double *u
     const int prev[2] = {c->rhs_shape, c->visc_shape};
     int best[2] = {prev[0], prev[1]};
     for (int i = 0; us_out && i < 2 * PRANDTL_SHAPES; i++) us_out[i] = -1.0;
-    // k_visc first (k_rhs reads its outputs), then k_rhs
+    // the viscous kernel first (the RHS kernel reads its outputs), then the RHS kernel
     for (int kern = PRANDTL_KERNEL_VISC; kern >= PRANDTL_KERNEL_RHS && !rc; kern--) {
         int &cur = kern == PRANDTL_KERNEL_RHS ? c->rhs_shape : c->visc_shape;
         double best_us = 0.0;
@@ -1259,7 +1259,7 @@ int prandtl_autotune(prandtl_ctx *c, const double *u, int *shapes_out, double *u
             if (us_out) us_out[kern * PRANDTL_SHAPES + sh] = us;
             if (!any || us < best_us) { best[kern] = sh; best_us = us; any = true; }
         }
-        // the winner stays in place, so k_rhs is timed after the best k_visc
+        // the winner stays in place, so the RHS kernel is timed after the best viscous one
         if (!rc) cur = best[kern];
         if (!rc && kern == PRANDTL_KERNEL_VISC && c->prm.parabolic) rc = visc_only(c, u, nullptr, s);
     }

@@ -38,10 +38,11 @@
 //  - The indicator's transforms run on the line threads: NP values in
 //    registers, NP^2 multiply-adds.
 //
-// Bound: FP64 issue and, next, HBM traffic; at three or four waves per SIMD
-// neither is hidden completely.  3-D N = 7, 32^3 elements, blended
-// Navier-Stokes: 3,025 vector instructions per wave, 0.53 ms of issue and 3 GB,
-// 0.55 ms at the copy rate, in 0.95 ms (two waves per SIMD: 1.16 times
+// Bound: at 3-D N = 3, 45 x 43 x 41 elements with Navier-Stokes terms, HBM: 0.96
+// GB, 0.21 ms at the 4.55 TB/s of a large copy, in 0.22 ms.  At 3-D N = 7, 32^3
+// elements, blended Navier-Stokes, FP64 issue and HBM together: 3,025 vector
+// instructions per wave, 0.53 ms of issue, and 2.6 GB, 0.58 ms at the copy rate, in
+// 0.99 ms at three waves per SIMD, which hide neither completely (two: 1.16 times
 // slower).  Against the kernel that took pairs as jobs, per right-hand side:
 // that case 3,475 -> 1,617 us (k_visc's 660 included); 2-D N = 3, 384^2
 // blended 172 -> 70; Euler 16^3 N = 7 279 -> 95, 28^3 N = 4 207 -> 125, 9x8x7

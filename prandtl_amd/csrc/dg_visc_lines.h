@@ -30,16 +30,17 @@
 //  D is applied in even-odd form (half the multiply-adds, and few enough
 //  entries for scalar registers), D^ as D and its boundary terms.
 //
-// Bound: latency at three to four waves per SIMD; at N = 7 1.8 GB of HBM
-// traffic (0.4 ms at the copy rate), 0.22 ms of vector issue and 0.16 ms of LDS
-// in 0.54 ms.  Against k_visc, which read a line's nodes once per node
+// Bound: HBM on large meshes: 0.72 GB, 0.16 ms at the 4.55 TB/s of a large copy,
+// in 0.17 ms at 3-D N = 3 45 x 43 x 41; 2.2 GB, 0.48 ms, in 0.55 at N = 7 32^3 (0.22
+// ms of vector issue, 0.16 ms of LDS).  At 16^3, all resident at once at three to
+// four waves per SIMD, latency.  Against k_visc, which read a line's nodes once per node
 // (240 LDS reads per node at N = 7, 80 here) and took four logarithms per node
 // and face point, per launch: 3-D N = 3 16^3 17.2 -> 12.2 us, 45 x 43 x 41 208
 // -> 170, N = 7 32^3 686 -> 540; mixed N = 3 16^3 15.6 (on the FP32 matrix
 // cores) -> 9.5.  With one trace per face point instead of two to read, k_rhs_l
 // takes 16.6 instead of 17.6, 242 instead of 250 and 980 instead of 1031.
-// Error against 64 bits, relative L2 of a right-hand side: N = 2..6 0.95 times
-// k_visc's, N = 7 1.02 times (8.6e-13); mixed 0.85 to 0.97 times.
+// Error against long double, relative L2 of a right-hand side of a fine mesh, next
+// to k_visc's: N = 4, 5 and 7 0.82 to 0.97 times; mixed, against FP64, 0.85 to 0.97 times.
 //
 // MIXED: the mixed-precision form, as k_visc's: v, T and the entropy variables,
 // shifted by their value at the element's node 0, are formed in FP64 and
